@@ -33,6 +33,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <shared_mutex>
 #include <string>
 #include <type_traits>
 #include <utility>
@@ -1529,6 +1530,8 @@ __global__ void __launch_bounds__(256) residual_kernel(const StepArgs<typename S
   step_cell<S, MODE>(a, sh, cells[k], st_rho, st_usqr, counted);
 }
 
+#include "olbgfx_pair.h"
+
 // ---------------------------------------------------------------------------
 // the ensemble kernel: one persistent launch advances one group of member
 // lattices by one step.  The work is a list of tiles (member, first core
@@ -1815,6 +1818,13 @@ olbgfx_status noalloc_scratch(double** ptr)
 
 }  // namespace
 
+// tiles of the two-step kernel (pair_tiles), a function of the lattice's extents
+struct PairPlan {
+  uint32_t threads = 0;  // 0: not chosen yet
+  uint32_t tz = 0, ty = 0, ntz = 0, nty = 0, xlen = 0, nwork = 0;
+  bool worth = false;
+};
+
 struct olbgfx_lattice {
   olbgfx_lattice_desc desc{};
   int elem = 4;               // bytes per stored population
@@ -1882,11 +1892,56 @@ struct olbgfx_lattice {
   uint32_t residual_n = 0;
   uint64_t split_version = ~0ull;
   bool split_enabled = true;         // olbgfx_set_split
+  // second set of populations, which passes of two steps write to: held from
+  // the first run of steps that takes them until the lattice is destroyed or
+  // an allocation needs the memory
+  void* pair_pop = nullptr;
+  int pair_device = 0;
+  PairPlan pair_plan;
+  bool pair_enabled = true;          // off while the tuner times single steps
 };
 
 namespace {
 
 bool is_f64(const olbgfx_lattice* L) { return L->desc.storage == OLBGFX_STORE_F64; }
+
+// Second population buffers are working memory: an allocation that fails takes
+// those of its device back and tries again.  Enqueueing pairs holds the lock
+// shared, taking buffers back holds it alone and waits for the device first.
+std::shared_mutex g_pair_use;
+std::mutex g_pair_list;
+std::vector<olbgfx_lattice*> g_pair_owners;
+
+void drop_pair_buffer(olbgfx_lattice* L)
+{
+  std::lock_guard<std::mutex> lock(g_pair_list);
+  g_pair_owners.erase(std::remove(g_pair_owners.begin(), g_pair_owners.end(), L), g_pair_owners.end());
+  (void)hipFree(L->pair_pop);
+  L->pair_pop = nullptr;
+}
+
+template <typename T>
+hipError_t device_alloc(T** ptr, size_t bytes)
+{
+  hipError_t e = hipMalloc(ptr, bytes);
+  int device = 0;
+  if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess) {
+    std::unique_lock<std::shared_mutex> alone(g_pair_use);
+    std::lock_guard<std::mutex> lock(g_pair_list);
+    (void)hipDeviceSynchronize();
+    for (size_t k = g_pair_owners.size(); k-- > 0;) {
+      olbgfx_lattice* L = g_pair_owners[k];
+      if (L->pair_device == device) {
+        (void)hipFree(L->pair_pop);
+        L->pair_pop = nullptr;
+        g_pair_owners.erase(g_pair_owners.begin() + (ptrdiff_t)k);
+      }
+    }
+    (void)hipGetLastError();
+    e = hipMalloc(ptr, bytes);
+  }
+  return e;
+}
 
 template <typename A>
 void fill_table(const olbgfx_lattice* L, DynEntry<A>* t)
@@ -2132,12 +2187,214 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
     }
   }
   if (!rest.empty()) {
-    HIP_TRY(hipMalloc(&L->residual_dev, sizeof(uint32_t) * rest.size()));
+    HIP_TRY(device_alloc(&L->residual_dev, sizeof(uint32_t) * rest.size()));
     HIP_TRY(hipMemcpy(L->residual_dev, rest.data(), sizeof(uint32_t) * rest.size(), hipMemcpyHostToDevice));
   }
   L->residual_n = (uint32_t)rest.size();
   L->split_id = dom;
   L->split_faces = faces;
+  return OLBGFX_OK;
+}
+
+// ---------------------------------------------------------------------------
+// runs of steps, two steps a pass (olbgfx_pair.h)
+
+// Workgroup size of the two-step kernel for this lattice, or 0 where single
+// steps are faster; mode is the kind of a uniform lattice or -1.  Two steps a
+// pass halve the traffic to HBM but do the first step of every tile's rim
+// twice, so they win where HBM bounds the single step: from 256 MiB of
+// populations, the size of the Infinity Cache (us a step, single / two a pass:
+// BGK 160^3 FP32 132 / 86, 512^3 FP32 4378 / 2765, FP16 2220 / 1752, BF16
+// 2249 / 1705; the porous channel 384x128x128 FP32 221 / 149; a closed cavity
+// 256^3 FP32 551 / 404, 200^3 FP64 515 / 375).  Below that size they win only
+// for uniform BGK, where the pass is short enough that the saved launch and
+// the saved round trip to the cache count: FP32 64^3 8.5 / 7.2, 101^3 27.5 /
+// 16.6, 128^3 47.2 / 47.2; FP64 64^3 14.3 / 11.9.  Masked cells in 2-byte
+// storage are bound by instruction issue and lose (porous channel FP16 124 /
+// 136).  1024 threads keep the rim small; 512 give more workgroups to small
+// lattices (101^3 FP32 16.6 against 18.0) and, in 2-byte storage, a second
+// workgroup on each CU, which pays for the larger rim in the largest lattices
+// (512^3 FP16 1752 against 1842) and for BF16 BGK (256^3 233 against 246),
+// whose kernel needs the fewest registers.
+uint32_t pair_threads(const olbgfx_lattice* L, int mode)
+{
+  const olbgfx_lattice_desc& D = L->desc;
+  const uint64_t cells = (uint64_t)D.nx * D.ny * D.nz;
+  const uint64_t bytes = (uint64_t)Q * L->stride * L->elem;
+  const bool beyond_cache = bytes >= (256ull << 20);
+  const bool bgk = mode == OLBGFX_BGK;
+  if (L->elem == 2) {
+    if (mode < 0 || !beyond_cache) {
+      return 0;
+    }
+    return cells >= (64u << 20) || (bgk && L->desc.storage == OLBGFX_STORE_BF16) ? 512 : 1024;
+  }
+  if (L->elem == 8) {
+    return beyond_cache || (bgk && bytes >= (48ull << 20)) ? 512 : 0;
+  }
+  if (bgk && cells >= 60000 && cells < 1500000) {
+    return 512;
+  }
+  return beyond_cache || (bgk && cells >= 1500000) ? 1024 : 0;
+}
+
+// the lattice's second set of populations; false where it cannot be had: the
+// stream is being captured, or it would take more than a quarter of the free
+// device memory
+bool prepare_pair(olbgfx_lattice* L, hipStream_t stream)
+{
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (!L->pair_pop) {
+    const size_t bytes = (size_t)Q * L->stride * L->elem;
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > free_bytes / 4 ||
+        hipMalloc(&L->pair_pop, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      L->pair_pop = nullptr;
+      return false;
+    }
+    (void)hipGetDevice(&L->pair_device);
+    std::lock_guard<std::mutex> lock(g_pair_list);
+    g_pair_owners.push_back(L);
+  }
+  return true;
+}
+
+// Tile and segment sizes: the product of the rounds the workgroups take on 256
+// CUs, the planes each sweeps (two of them its rim, one to start), and the
+// cost of a plane, which is that of its cells plus, where HBM bounds it, of
+// its rows (every row of a tile begins and ends inside a cache line that it
+// shares with the next tile: 512^3 FP32 takes 2.70 ms a step in tiles 128 wide
+// and 3.16 in tiles 64 wide, though these have the smaller rim).  Rows that are
+// no multiple of 64 split waves across rows: 1.12 times.  Segments of more
+// than 16 planes lose the cache lines that neighbouring tiles share as the
+// tiles drift apart (512^3 FP32: 2.70, 2.82, 3.05 and 3.27 ms with 16, 32, 64
+// and 128 planes).
+//
+// Lattices one or a few cells thin, whose planes the best tiles fill to less
+// than 0.4 or which have fewer than 4 planes, keep single steps: rims would be
+// most of the work (the tiles of 512^3 are filled to 0.60 in FP32).
+void pair_tiles(PairPlan& plan, const olbgfx_lattice* L, uint32_t threads)
+{
+  const olbgfx_lattice_desc& D = L->desc;
+  const uint32_t pad2 = D.periodic[0] ? 0 : 2 * (uint32_t)D.padding;
+  const uint32_t dx = D.nx + pad2, dy = D.ny + pad2, dz = D.nz + pad2;
+  const uint32_t slots = 256 * 1024 / threads;
+  const double row = L->elem > 2 && (uint64_t)Q * L->stride * L->elem >= (256ull << 20) ? 128 : 32;
+  double best = 0;
+  for (uint32_t tz = 3; tz <= std::min(threads / 3, dz + 2); ++tz) {
+    const uint32_t ty = std::min(threads / tz, dy + 2);
+    const uint32_t ntz = (dz + tz - 3) / (tz - 2), nty = (dy + ty - 3) / (ty - 2);
+    for (uint32_t len = 1; len <= 16; ++len) {
+      const uint64_t work = (uint64_t)ntz * nty * ((dx + len - 1) / len);
+      const double cost = (double)((work + slots - 1) / slots) * (std::min(len, dx) + 3) *
+                          (threads + row * ty) * (tz % 64 ? 1.12 : 1.0);
+      if (best == 0 || cost <= best) {
+        best = cost;
+        plan.tz = tz;
+        plan.ty = ty;
+        plan.ntz = ntz;
+        plan.nty = nty;
+        plan.xlen = len;
+        plan.nwork = (uint32_t)work;
+      }
+    }
+  }
+  plan.worth = dx >= 4 && (double)dy * dz >= 0.4 * ((double)plan.ntz * plan.nty * threads);
+  plan.threads = threads;
+}
+
+template <typename S, uint32_t NT, int MODE, bool PERIODIC>
+void launch_pair_form(bool src_ring, bool dst_ring, dim3 grid, hipStream_t stream,
+                      const PairArgs<typename Storage<S>::A>& p)
+{
+  if (src_ring) {
+    pair_kernel<S, NT, MODE, PERIODIC, true, false><<<grid, NT, 0, stream>>>(p);
+  } else if (dst_ring) {
+    pair_kernel<S, NT, MODE, PERIODIC, false, true><<<grid, NT, 0, stream>>>(p);
+  } else {
+    pair_kernel<S, NT, MODE, PERIODIC, false, false><<<grid, NT, 0, stream>>>(p);
+  }
+}
+
+template <typename S, uint32_t NT>
+void launch_pair_mode(int mode, bool periodic, bool src_ring, bool dst_ring, dim3 grid, hipStream_t stream,
+                      const PairArgs<typename Storage<S>::A>& p)
+{
+  if (periodic) {
+    switch (mode) {
+    case OLBGFX_BGK:
+      return launch_pair_form<S, NT, OLBGFX_BGK, true>(src_ring, dst_ring, grid, stream, p);
+    case OLBGFX_FORCED_TRT:
+      return launch_pair_form<S, NT, OLBGFX_FORCED_TRT, true>(src_ring, dst_ring, grid, stream, p);
+    case OLBGFX_SMAGORINSKY_BGK:
+      return launch_pair_form<S, NT, OLBGFX_SMAGORINSKY_BGK, true>(src_ring, dst_ring, grid, stream, p);
+    default:
+      break;
+    }
+  }
+  // masked cells are updated in pairs in these forms only (pair_threads)
+  if constexpr ((sizeof(S) == 4 && NT == 1024) || sizeof(S) == 8) {
+    if (periodic) {
+      launch_pair_form<S, NT, -1, true>(src_ring, dst_ring, grid, stream, p);
+    } else {
+      launch_pair_form<S, NT, -1, false>(src_ring, dst_ring, grid, stream, p);
+    }
+  }
+}
+
+// two steps from src to dst; shift: the source offsets, dshift those of the
+// destination after the first of the two steps
+template <typename S>
+olbgfx_status launch_pair(olbgfx_lattice* L, const StepArgs<typename Storage<S>::A>& a, int mode, void* dst,
+                          const uint32_t (&dshift)[Q], bool src_ring, bool dst_ring, hipStream_t stream)
+{
+  PairArgs<typename Storage<S>::A> p;
+  p.a = a;
+  p.dst = dst;
+  for (int i = 0; i < Q; ++i) p.dshift[i] = dshift[i];
+  const olbgfx_lattice_desc& D = L->desc;
+  const bool periodic = D.periodic[0] != 0;
+  const int pad2 = periodic ? 0 : 2 * D.padding;
+  p.dx = D.nx + pad2;
+  p.dy = D.ny + pad2;
+  p.dz = D.nz + pad2;
+  p.plane = L->py * L->pz;
+  // flat layout: on periodic lattices rows of a whole number of cache lines
+  // where the buffer has room for that, and the rows of the 19 populations
+  // side by side where the offsets within a plane then fit in 32 bits; the
+  // padded block as it is on closed ones
+  const uint32_t line = 128 / sizeof(S);
+  uint32_t pitch = (uint32_t)p.dz;
+  const uint32_t aligned = (pitch + line - 1) / line * line;
+  if (periodic && (uint64_t)p.dx * p.dy * aligned <= L->stride) {
+    pitch = aligned;
+  }
+  const bool rows = periodic && (uint64_t)p.dy * pitch * Q * sizeof(S) < (1ull << 32);
+  p.fq = rows ? pitch : (uint32_t)L->stride;
+  p.fy = rows ? pitch * Q : pitch;
+  p.fx = (uint32_t)p.dy * p.fy;
+  const PairPlan& plan = L->pair_plan;
+  p.tz = plan.tz;
+  p.ty = plan.ty;
+  p.ntz = plan.ntz;
+  p.nty = plan.nty;
+  p.xlen = plan.xlen;
+  p.nwork = plan.nwork;
+  p.per_xcd = (p.nwork + 7) / 8;
+  const dim3 grid(8 * p.per_xcd);
+  if constexpr (sizeof(S) == 8) {
+    launch_pair_mode<S, 512>(mode, periodic, src_ring, dst_ring, grid, stream, p);
+  } else if (plan.threads == 512) {
+    launch_pair_mode<S, 512>(mode, periodic, src_ring, dst_ring, grid, stream, p);
+  } else {
+    launch_pair_mode<S, 1024>(mode, periodic, src_ring, dst_ring, grid, stream, p);
+  }
+  HIP_TRY(hipGetLastError());
   return OLBGFX_OK;
 }
 
@@ -2158,7 +2415,7 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
       HIP_TRY(hipFree(L->stats_partial));
       L->stats_partial = nullptr;
     }
-    HIP_TRY(hipMalloc(&L->stats_partial, 4 * sizeof(double) * (size_t)a.nblocks));
+    HIP_TRY(device_alloc(&L->stats_partial, 4 * sizeof(double) * (size_t)a.nblocks));
     L->stats_capacity = a.nblocks;
     a.stats = L->stats_partial;
   }
@@ -2178,7 +2435,48 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
   }
   const int dominant =
       split ? (L->split_faces ? kWithFaces : 0) + L->table[L->split_id].kind : mode;
-  for (uint32_t k = 0; k < steps; ++k) {
+  uint32_t first = 0;
+  // Two steps a pass, four steps at a time so that the populations end where
+  // they began: the rings of L->pop; the passes between write the flat layout
+  // to the second buffer and to L->pop in turn.  The statistics are those of
+  // the last step, which runs alone.
+  const bool all = a.periodic == 7, none = a.periodic == 0;  // mixed axes take single steps
+  const bool pair_kind = all && (mode == OLBGFX_BGK || mode == OLBGFX_FORCED_TRT || mode == OLBGFX_SMAGORINSKY_BGK);
+  const int pair_mode = pair_kind ? mode : -1;
+  uint32_t threads = 0;
+  if (L->pair_enabled && (all || none) && steps > 0 && !L->boundary_kinds && L->bz_n == 0 && L->bzv_n == 0 &&
+      L->inflight_limit == 0 && mode != OLBGFX_NO_DYNAMICS) {
+    threads = pair_threads(L, pair_mode);
+    if (threads > 0 && L->pair_plan.threads != threads) {
+      pair_tiles(L->pair_plan, L, threads);
+    }
+  }
+  const uint32_t in_pairs = (L->stats_on ? steps - 1 : steps) / 4 * 4;
+  if (threads > 0 && in_pairs > 0 && L->pair_plan.worth) {
+    std::shared_lock<std::shared_mutex> use(g_pair_use);
+    const uint32_t end = prepare_pair(L, stream) ? in_pairs : 0;
+    auto advance = [&](uint32_t (&s)[Q]) {
+      for (int i = 0; i < Q; ++i) {
+        const uint64_t v = (uint64_t)s[i] + (uint64_t)L->dmod[i];
+        s[i] = (uint32_t)(v >= L->count ? v - L->count : v);
+      }
+    };
+    void* rings[2] = {L->pop, L->pair_pop};
+    uint32_t dshift[Q];
+    for (; first < end; first += 2) {
+      a.pop = rings[0];
+      for (int i = 0; i < Q; ++i) a.shift[i] = L->shift[i];
+      advance(L->shift);
+      for (int i = 0; i < Q; ++i) dshift[i] = L->shift[i];
+      advance(L->shift);
+      if (launch_pair<S>(L, a, pair_mode, rings[1], dshift, first == 0, first + 2 == end, stream) != OLBGFX_OK) {
+        return OLBGFX_ERR_HIP;
+      }
+      std::swap(rings[0], rings[1]);
+    }
+    a.pop = L->pop;
+  }
+  for (uint32_t k = first; k < steps; ++k) {
     for (int i = 0; i < Q; ++i) a.shift[i] = L->shift[i];
     if (L->stats_on) {
       launch_mode<S, true>(mode, grid, block, L->lds_reserve, stream, a);
@@ -2231,7 +2529,7 @@ template <typename S, typename H>
 olbgfx_status transfer_pop(olbgfx_lattice* L, void* host, bool to_device)
 {
   H* tmp = nullptr;
-  HIP_TRY(hipMalloc(&tmp, sizeof(H) * (size_t)L->count));
+  HIP_TRY(device_alloc(&tmp, sizeof(H) * (size_t)L->count));
   const dim3 block(256);
   const dim3 grid((L->count + 255) / 256);
   olbgfx_status st = OLBGFX_OK;
@@ -2309,7 +2607,7 @@ olbgfx_status upload_values(olbgfx_lattice* L, void** dst, int32_t vt, const voi
     }
   }
   if (!*dst) {
-    HIP_TRY(hipMalloc(dst, n * esz));
+    HIP_TRY(device_alloc(dst, n * esz));
   }
   HIP_TRY(hipMemcpy(*dst, conv.data(), n * esz, hipMemcpyHostToDevice));
   return OLBGFX_OK;
@@ -2493,7 +2791,7 @@ olbgfx_status prepare_boundary(olbgfx_lattice* L)
   }
   L->refresh_n = (uint32_t)(pairs.size() / 2);
   if (!pairs.empty()) {
-    HIP_TRY(hipMalloc(&L->refresh_dev, sizeof(uint32_t) * pairs.size()));
+    HIP_TRY(device_alloc(&L->refresh_dev, sizeof(uint32_t) * pairs.size()));
     HIP_TRY(hipMemcpy(L->refresh_dev, pairs.data(), sizeof(uint32_t) * pairs.size(), hipMemcpyHostToDevice));
   }
   if (L->post_dev) {
@@ -2504,7 +2802,7 @@ olbgfx_status prepare_boundary(olbgfx_lattice* L)
   L->post_corners = (uint32_t)corners.size();
   if (!edges.empty() || !corners.empty()) {
     edges.insert(edges.end(), corners.begin(), corners.end());
-    HIP_TRY(hipMalloc(&L->post_dev, sizeof(uint32_t) * edges.size()));
+    HIP_TRY(device_alloc(&L->post_dev, sizeof(uint32_t) * edges.size()));
     HIP_TRY(hipMemcpy(L->post_dev, edges.data(), sizeof(uint32_t) * edges.size(), hipMemcpyHostToDevice));
   }
   if (L->fd_dev) {
@@ -2518,9 +2816,9 @@ olbgfx_status prepare_boundary(olbgfx_lattice* L)
   L->fd_n = (uint32_t)fd.size();
   if (!fd.empty()) {
     const size_t value = L->desc.storage == OLBGFX_STORE_F64 ? sizeof(double) : sizeof(float);
-    HIP_TRY(hipMalloc(&L->fd_dev, sizeof(uint32_t) * fd.size()));
+    HIP_TRY(device_alloc(&L->fd_dev, sizeof(uint32_t) * fd.size()));
     HIP_TRY(hipMemcpy(L->fd_dev, fd.data(), sizeof(uint32_t) * fd.size(), hipMemcpyHostToDevice));
-    HIP_TRY(hipMalloc(&L->fd_out, value * Q * fd.size()));
+    HIP_TRY(device_alloc(&L->fd_out, value * Q * fd.size()));
   }
   L->boundary_kinds = used;
   L->boundary_version = L->version;
@@ -2598,16 +2896,16 @@ olbgfx_status olbgfx_lattice_create(const olbgfx_lattice_desc* desc, olbgfx_latt
     return s;
   };
   const size_t bytes = (size_t)Q * L->stride * L->elem;
-  if (hipMalloc(&L->pop, bytes) != hipSuccess) {
+  if (device_alloc(&L->pop, bytes) != hipSuccess) {
     return cleanup(fail(OLBGFX_ERR_NOMEM, "population allocation failed"));
   }
   if (hipMemset(L->pop, 0, bytes) != hipSuccess ||
-      hipMalloc(&L->mask, count) != hipSuccess || hipMemset(L->mask, 0, count) != hipSuccess ||
-      hipMalloc(&L->shift_dev, sizeof(L->shift)) != hipSuccess ||
+      device_alloc(&L->mask, count) != hipSuccess || hipMemset(L->mask, 0, count) != hipSuccess ||
+      device_alloc(&L->shift_dev, sizeof(L->shift)) != hipSuccess ||
       hipMemset(L->shift_dev, 0, sizeof(L->shift)) != hipSuccess ||
-      hipMalloc(&L->kinds_dev, sizeof(int32_t) * 256) != hipSuccess ||
+      device_alloc(&L->kinds_dev, sizeof(int32_t) * 256) != hipSuccess ||
       hipMemset(L->kinds_dev, 0, sizeof(int32_t) * 256) != hipSuccess ||
-      hipMalloc(&L->stats_out, 4 * sizeof(double)) != hipSuccess ||
+      device_alloc(&L->stats_out, 4 * sizeof(double)) != hipSuccess ||
       hipMemset(L->stats_out, 0, 4 * sizeof(double)) != hipSuccess) {
     return cleanup(fail(OLBGFX_ERR_NOMEM, "device allocation failed"));
   }
@@ -2641,6 +2939,7 @@ olbgfx_status olbgfx_lattice_destroy(olbgfx_lattice* L)
   hipFree(L->stats_partial);
   hipFree(L->stats_out);
   hipFree(L->residual_dev);
+  drop_pair_buffer(L);
   for (hipEvent_t e : L->inflight_events) {
     hipEventDestroy(e);
   }
@@ -2809,7 +3108,7 @@ olbgfx_status olbgfx_set_cell_normals(olbgfx_lattice* L, const int8_t* normals)
   }
   L->host_normals.assign(normals, normals + 3 * (size_t)L->count);
   if (!L->normal_dev) {
-    HIP_TRY(hipMalloc(&L->normal_dev, L->count));
+    HIP_TRY(device_alloc(&L->normal_dev, L->count));
   }
   HIP_TRY(hipMemcpy(L->normal_dev, codes.data(), L->count, hipMemcpyHostToDevice));
   return OLBGFX_OK;
@@ -2925,13 +3224,13 @@ olbgfx_status set_bouzidi_list(olbgfx_lattice* L, int64_t n, const int64_t* cell
     return out;
   };
   const std::vector<char> qa = direction_major(qd);
-  HIP_TRY(hipMalloc(&dev_cells, sizeof(uint32_t) * ids.size()));
-  HIP_TRY(hipMalloc(&dev_q, qa.size()));
+  HIP_TRY(device_alloc(&dev_cells, sizeof(uint32_t) * ids.size()));
+  HIP_TRY(device_alloc(&dev_q, qa.size()));
   HIP_TRY(hipMemcpy(dev_cells, ids.data(), sizeof(uint32_t) * ids.size(), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(dev_q, qa.data(), qa.size(), hipMemcpyHostToDevice));
   if (vel) {
     const std::vector<char> va = direction_major(vd);
-    HIP_TRY(hipMalloc(&dev_v, va.size()));
+    HIP_TRY(device_alloc(&dev_v, va.size()));
     HIP_TRY(hipMemcpy(dev_v, va.data(), va.size(), hipMemcpyHostToDevice));
   }
   dev_n = (uint32_t)n;
@@ -3015,8 +3314,8 @@ olbgfx_status olbgfx_ini_equilibrium(olbgfx_lattice* L, const uint8_t* sel, int3
   void* d_u = nullptr;
   uint8_t* d_sel = nullptr;
   olbgfx_status st = OLBGFX_OK;
-  if (hipMalloc(&d_rho, n * vs) != hipSuccess || hipMalloc(&d_u, 3 * n * vs) != hipSuccess ||
-      (sel && hipMalloc(&d_sel, n) != hipSuccess)) {
+  if (device_alloc(&d_rho, n * vs) != hipSuccess || device_alloc(&d_u, 3 * n * vs) != hipSuccess ||
+      (sel && device_alloc(&d_sel, n) != hipSuccess)) {
     st = fail(OLBGFX_ERR_NOMEM, "temporary allocation failed");
   }
   if (st == OLBGFX_OK &&
@@ -3135,7 +3434,7 @@ olbgfx_status olbgfx_reduce_moments(olbgfx_lattice* L, double out[8], void* stre
   const uint64_t ncore = (uint64_t)D.nx * D.ny * D.nz;
   const uint32_t nb = (uint32_t)((ncore + 255) / 256);
   double* partial = nullptr;
-  HIP_TRY(hipMalloc(&partial, 8 * sizeof(double) * (size_t)nb));
+  HIP_TRY(device_alloc(&partial, 8 * sizeof(double) * (size_t)nb));
   hipStream_t s = (hipStream_t)stream;
   HIP_TRY(hipStreamSynchronize(s));
   if (sync_shifts(L) != OLBGFX_OK) {
@@ -3233,8 +3532,8 @@ olbgfx_status olbgfx_compute_rho_u(olbgfx_lattice* L, int32_t vt, void* rho, voi
   const size_t vs = value_size(vt);
   void* d_rho = nullptr;
   void* d_u = nullptr;
-  HIP_TRY(hipMalloc(&d_rho, n * vs));
-  if (hipMalloc(&d_u, 3 * n * vs) != hipSuccess) {
+  HIP_TRY(device_alloc(&d_rho, n * vs));
+  if (device_alloc(&d_u, 3 * n * vs) != hipSuccess) {
     hipFree(d_rho);
     return fail(OLBGFX_ERR_NOMEM, "temporary allocation failed");
   }
@@ -3464,23 +3763,23 @@ olbgfx_status ensemble_prepare(olbgfx_ensemble* E, bool force)
     E->groups.push_back(g);
   }
   if (!E->args_dev) {
-    HIP_TRY(hipMalloc(&E->args_dev, sizeof(StepArgs<A>) * m));
-    HIP_TRY(hipMalloc(&E->shift_ptrs_dev, sizeof(uint32_t*) * m));
-    HIP_TRY(hipMalloc(&E->dmod_dev, sizeof(uint32_t) * m * Q));
-    HIP_TRY(hipMalloc(&E->counts_dev, sizeof(uint32_t) * m));
+    HIP_TRY(device_alloc(&E->args_dev, sizeof(StepArgs<A>) * m));
+    HIP_TRY(device_alloc(&E->shift_ptrs_dev, sizeof(uint32_t*) * m));
+    HIP_TRY(device_alloc(&E->dmod_dev, sizeof(uint32_t) * m * Q));
+    HIP_TRY(device_alloc(&E->counts_dev, sizeof(uint32_t) * m));
   }
   if (tiles.size() > E->tiles_capacity) {
     if (E->tiles_dev) {
       HIP_TRY(hipFree(E->tiles_dev));
     }
-    HIP_TRY(hipMalloc(&E->tiles_dev, sizeof(Tile) * tiles.size()));
+    HIP_TRY(device_alloc(&E->tiles_dev, sizeof(Tile) * tiles.size()));
     E->tiles_capacity = (uint32_t)tiles.size();
   }
   if (E->groups.size() > E->counters_capacity) {
     if (E->counters_dev) {
       HIP_TRY(hipFree(E->counters_dev));
     }
-    HIP_TRY(hipMalloc(&E->counters_dev, sizeof(uint32_t) * E->groups.size()));
+    HIP_TRY(device_alloc(&E->counters_dev, sizeof(uint32_t) * E->groups.size()));
     E->counters_capacity = (uint32_t)E->groups.size();
   }
   // counters start at zero; the kernels leave them at zero (no launch of
@@ -4017,7 +4316,7 @@ olbgfx_status olbgfx_halo_buffer_create(const olbgfx_lattice* L, int32_t axis, v
     return fail(OLBGFX_ERR_INVALID, "null argument or axis outside [0, 2]");
   }
   *device_buffer = nullptr;
-  if (hipMalloc(device_buffer, std::max<uint64_t>(bytes, 256)) != hipSuccess) {
+  if (device_alloc(device_buffer, std::max<uint64_t>(bytes, 256)) != hipSuccess) {
     (void)hipGetLastError();
     *device_buffer = nullptr;
     return fail(OLBGFX_ERR_NOMEM, "halo buffer allocation failed");
@@ -4152,7 +4451,7 @@ olbgfx_status olbgfx_cell_list_create(const olbgfx_lattice* L, const uint32_t* c
   list->n = n;
   list->count = L->count;
   if (n > 0) {
-    if (hipMalloc(&list->cells, sizeof(uint32_t) * n) != hipSuccess) {
+    if (device_alloc(&list->cells, sizeof(uint32_t) * n) != hipSuccess) {
       (void)hipGetLastError();
       delete list;
       return fail(OLBGFX_ERR_NOMEM, "cell list allocation failed");
@@ -4205,7 +4504,7 @@ olbgfx_status olbgfx_device_buffer_create(uint64_t bytes, void** device_buffer)
     return fail(OLBGFX_ERR_INVALID, "null argument");
   }
   *device_buffer = nullptr;
-  if (hipMalloc(device_buffer, std::max<uint64_t>(bytes, 256)) != hipSuccess) {
+  if (device_alloc(device_buffer, std::max<uint64_t>(bytes, 256)) != hipSuccess) {
     (void)hipGetLastError();
     *device_buffer = nullptr;
     return fail(OLBGFX_ERR_NOMEM, "device buffer allocation failed");
@@ -4252,7 +4551,7 @@ olbgfx_status save_state(olbgfx_lattice* L, hipStream_t stream, SavedState& out)
 {
   out.L = L;
   const size_t bytes = (size_t)Q * L->stride * L->elem;
-  if (hipMalloc(&out.pop, bytes) != hipSuccess) {
+  if (device_alloc(&out.pop, bytes) != hipSuccess) {
     (void)hipGetLastError();
     out.pop = nullptr;
     return fail(OLBGFX_ERR_NOMEM, "not enough device memory to keep the lattice state while tuning");
@@ -4462,6 +4761,9 @@ olbgfx_status olbgfx_autotune_lattice(olbgfx_lattice* L, uint32_t steps, const o
   hipStream_t s = (hipStream_t)stream;
   std::vector<SavedState> saved(1);
   olbgfx_status st = save_state(L, s, saved[0]);
+  // the choices are for single steps
+  const bool pairs = L->pair_enabled;
+  L->pair_enabled = false;
   auto trial = [&](uint32_t b, uint32_t w, int32_t o) -> olbgfx_status {
     olbgfx_status r = olbgfx_set_launch(L, b, w);
     if (r == OLBGFX_OK) r = olbgfx_set_block_order(L, o);
@@ -4494,6 +4796,7 @@ olbgfx_status olbgfx_autotune_lattice(olbgfx_lattice* L, uint32_t steps, const o
       }
     }
   }
+  L->pair_enabled = pairs;
   if (saved[0].pop) {
     const std::string err = st == OLBGFX_OK ? std::string() : g_error;
     const olbgfx_status rs = restore_state(saved[0], s);
