@@ -1847,6 +1847,7 @@ struct olbgfx_lattice {
   bool stats_on = false;
   bool stats_valid = false;
   int32_t uniform_id = 0;     // all cells start with id 0 = NoDynamics
+  uint32_t core_ids = 1;      // bit k: some core cell has id k
   uint32_t block_threads = 256;
   uint32_t lds_reserve = 0;    // dynamic LDS per block that limits occupancy
   int32_t xcd_run_log2 = -1;   // block order of the step kernel (olbgfx_set_block_order)
@@ -2218,13 +2219,14 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
 // whose kernel needs the fewest registers.
 uint32_t pair_threads(const olbgfx_lattice* L, int mode)
 {
+  const bool masked = mode < 0 || mode >= kWithWalls;
   const olbgfx_lattice_desc& D = L->desc;
   const uint64_t cells = (uint64_t)D.nx * D.ny * D.nz;
   const uint64_t bytes = (uint64_t)Q * L->stride * L->elem;
   const bool beyond_cache = bytes >= (256ull << 20);
   const bool bgk = mode == OLBGFX_BGK;
   if (L->elem == 2) {
-    if (mode < 0 || !beyond_cache) {
+    if (masked || !beyond_cache) {
       return 0;
     }
     return cells >= (64u << 20) || (bgk && L->desc.storage == OLBGFX_STORE_BF16) ? 512 : 1024;
@@ -2339,10 +2341,18 @@ void launch_pair_mode(int mode, bool periodic, bool src_ring, bool dst_ring, dim
   }
   // masked cells are updated in pairs in these forms only (pair_threads)
   if constexpr ((sizeof(S) == 4 && NT == 1024) || sizeof(S) == 8) {
+    auto masked = [&](auto per) {
+      constexpr bool P = decltype(per)::value;
+      if (mode == kWithWalls + OLBGFX_BGK) {
+        launch_pair_form<S, NT, kWithWalls + OLBGFX_BGK, P>(src_ring, dst_ring, grid, stream, p);
+      } else {
+        launch_pair_form<S, NT, -1, P>(src_ring, dst_ring, grid, stream, p);
+      }
+    };
     if (periodic) {
-      launch_pair_form<S, NT, -1, true>(src_ring, dst_ring, grid, stream, p);
+      masked(std::true_type{});
     } else {
-      launch_pair_form<S, NT, -1, false>(src_ring, dst_ring, grid, stream, p);
+      masked(std::false_type{});
     }
   }
 }
@@ -2398,6 +2408,23 @@ olbgfx_status launch_pair(olbgfx_lattice* L, const StepArgs<typename Storage<S>:
   return OLBGFX_OK;
 }
 
+// kWithWalls + BGK where the core cells hold no other kind besides bounce-back
+// and NoDynamics, -1 otherwise.  That kernel has one bulk kind and its
+// parameters in scalar registers (us a step, against the kernel of every kind:
+// cavity 160^3 FP32 94 / 99, 256^3 387 / 404, 160^3 FP64 180 / 199); the same
+// for ForcedTRT was slower (porous channel FP32 154 / 149, 160^3 FP64 223 / 207).
+int wall_mode(const olbgfx_lattice* L)
+{
+  for (int id = 0; id < OLBGFX_MAX_DYNAMICS; ++id) {
+    const int k = L->table[id].kind;
+    if ((L->core_ids >> id & 1) && k != OLBGFX_BGK && k != OLBGFX_NO_DYNAMICS && k != OLBGFX_BOUNCE_BACK &&
+        k != OLBGFX_BOUNCE_BACK_VELOCITY) {
+      return -1;
+    }
+  }
+  return kWithWalls + OLBGFX_BGK;
+}
+
 template <typename S>
 olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream)
 {
@@ -2442,7 +2469,7 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
   // the last step, which runs alone.
   const bool all = a.periodic == 7, none = a.periodic == 0;  // mixed axes take single steps
   const bool pair_kind = all && (mode == OLBGFX_BGK || mode == OLBGFX_FORCED_TRT || mode == OLBGFX_SMAGORINSKY_BGK);
-  const int pair_mode = pair_kind ? mode : -1;
+  const int pair_mode = pair_kind ? mode : wall_mode(L);
   uint32_t threads = 0;
   if (L->pair_enabled && (all || none) && steps > 0 && !L->boundary_kinds && L->bz_n == 0 && L->bzv_n == 0 &&
       L->inflight_limit == 0 && mode != OLBGFX_NO_DYNAMICS) {
@@ -2621,25 +2648,21 @@ olbgfx_status check(const olbgfx_lattice* L)
   return OLBGFX_OK;
 }
 
+// the ids of the core cells, and the id they share if they do
 void recompute_uniform(olbgfx_lattice* L)
 {
   const olbgfx_lattice_desc& D = L->desc;
-  int id = -2;
-  for (int x = 0; x < D.nx && id != -1; ++x) {
-    for (int y = 0; y < D.ny && id != -1; ++y) {
+  uint32_t ids = 0;
+  for (int x = 0; x < D.nx; ++x) {
+    for (int y = 0; y < D.ny; ++y) {
       const size_t base = ((size_t)(x + D.padding) * L->py + (y + D.padding)) * L->pz + D.padding;
       for (int z = 0; z < D.nz; ++z) {
-        const int v = L->host_mask[base + z];
-        if (id == -2) {
-          id = v;
-        } else if (v != id) {
-          id = -1;
-          break;
-        }
+        ids |= 1u << L->host_mask[base + z];
       }
     }
   }
-  L->uniform_id = id < 0 ? -1 : id;
+  L->core_ids = ids;
+  L->uniform_id = (ids & (ids - 1)) == 0 ? __builtin_ctz(ids) : -1;
 }
 
 // find the LocalVelocity cells and the post-processed edges and corners;

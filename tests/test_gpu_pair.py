@@ -115,6 +115,24 @@ def test_masked_runs(storage, periodic, extent, padding):
     b.close()
 
 
+@pytest.mark.parametrize("storage,periodic,extent,padding", MASKED)
+def test_bgk_with_bounce_back_runs(storage, periodic, extent, padding):
+    """two BGK slots, bounce-back, a moving wall and NoDynamics cells: the
+    kernel with one bulk kind"""
+    print(f"[pair] walls {storage} periodic={periodic} {extent} p{padding}", flush=True)
+    rng = np.random.default_rng(12)
+    slots = {1: Dynamics(BGK, omega=1 / 0.61), 2: Dynamics(BGK, omega=1 / 0.9), 3: Dynamics(BOUNCE_BACK),
+             4: Dynamics(NO_DYNAMICS), 6: Dynamics(BOUNCE_BACK_VELOCITY, wall_velocity=(0.02, 0.0, -0.01))}
+    mask = rng.choice(np.array([1, 1, 1, 2, 3, 4, 6], dtype=np.uint8), _padded(extent, padding))
+    a, b = _pair(extent, padding, periodic, storage, mask, slots)
+    a.collide_and_stream(8)
+    for _ in range(8):
+        b.collide_and_stream(1)
+    _compare(a, b, storage, not periodic)
+    a.close()
+    b.close()
+
+
 def test_lattice_of_an_ensemble_keeps_its_buffer():
     """a member that runs on its own between ensemble steps"""
     from openlb_amd import Ensemble
