@@ -1622,18 +1622,28 @@ __global__ void advance_shifts(uint32_t* const* shifts, const uint32_t* dmod, co
   }
 }
 
-// sums the per-block statistics in a fixed order (deterministic)
-__global__ void __launch_bounds__(256) stats_finalize(const double* partial, uint32_t nblocks,
-                                                      double* out)
+// Sums the per-block statistics in a fixed order (deterministic).  Block g of G
+// takes the partials [g * chunk, (g + 1) * chunk); one block takes all of up to
+// kStatsChunk, more go through a second launch over the G sums.  One block over
+// everything took 117 us on the 65536 partials of 256^3, a third of the step,
+// because its 256 threads each waited for 256 loads in turn; two launches with
+// a chunk a block take 9 us.
+constexpr uint32_t kStatsChunk = 2048;
+constexpr uint32_t kStatsThreads = 512;
+
+__global__ void __launch_bounds__(kStatsThreads) stats_finalize(const double* partial, uint32_t n, uint32_t chunk,
+                                                                double* out)
 {
+  const uint32_t first = blockIdx.x * chunk, last = min(first + chunk, n);
   double c = 0, r = 0, e = 0, m = 0;
-  for (uint32_t k = threadIdx.x; k < nblocks; k += blockDim.x) {
+#pragma unroll 4
+  for (uint32_t k = first + threadIdx.x; k < last; k += kStatsThreads) {
     c += partial[4 * (size_t)k + 0];
     r += partial[4 * (size_t)k + 1];
     e += partial[4 * (size_t)k + 2];
     m = fmax(m, partial[4 * (size_t)k + 3]);
   }
-  block_reduce4(c, r, e, m, out, true);
+  block_reduce4(c, r, e, m, out + 4 * (size_t)blockIdx.x, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -1842,7 +1852,7 @@ struct olbgfx_lattice {
   void* cell_rho = nullptr;
   void* cell_force = nullptr;
   double* stats_partial = nullptr;
-  double* stats_out = nullptr;
+  double* stats_out = nullptr;   // pinned host memory that the device writes (4 doubles)
   uint32_t stats_capacity = 0;
   bool stats_on = false;
   bool stats_valid = false;
@@ -2210,13 +2220,16 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
 // 256^3 FP32 551 / 404, 200^3 FP64 515 / 375).  Below that size they win only
 // for uniform BGK, where the pass is short enough that the saved launch and
 // the saved round trip to the cache count: FP32 64^3 8.5 / 7.2, 101^3 27.5 /
-// 16.6, 128^3 47.2 / 47.2; FP64 64^3 14.3 / 11.9.  Masked cells in 2-byte
-// storage are bound by instruction issue and lose (porous channel FP16 124 /
-// 136).  1024 threads keep the rim small; 512 give more workgroups to small
-// lattices (101^3 FP32 16.6 against 18.0) and, in 2-byte storage, a second
-// workgroup on each CU, which pays for the larger rim in the largest lattices
-// (512^3 FP16 1752 against 1842) and for BF16 BGK (256^3 233 against 246),
-// whose kernel needs the fewest registers.
+// 16.6, 140^3 64.5 / 56.4, but 128^3 47.2 / 48.3 in runs of 8 steps; FP64 64^3
+// 14.3 / 11.9.  Masked cells and
+// Smagorinsky BGK in 2-byte storage are bound by instruction issue: the former
+// lose (porous channel FP16 124 / 133), the latter gain 7 % in long runs and
+// lose 8 % in runs of 8 steps, whose first and last pass convert the layout.
+// 1024 threads keep the rim small; 512 give more workgroups to small lattices
+// (101^3 FP32 16.6 against 18.0) and, in 2-byte storage, a second workgroup on
+// each CU, which pays for the larger rim in the largest lattices (512^3 FP16
+// 1752 against 1842) and for BF16 BGK (256^3 233 against 246), whose kernel
+// needs the fewest registers.
 uint32_t pair_threads(const olbgfx_lattice* L, int mode)
 {
   const bool masked = mode < 0 || mode >= kWithWalls;
@@ -2226,7 +2239,7 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
   const bool beyond_cache = bytes >= (256ull << 20);
   const bool bgk = mode == OLBGFX_BGK;
   if (L->elem == 2) {
-    if (masked || !beyond_cache) {
+    if (masked || mode == OLBGFX_SMAGORINSKY_BGK || !beyond_cache) {
       return 0;
     }
     return cells >= (64u << 20) || (bgk && L->desc.storage == OLBGFX_STORE_BF16) ? 512 : 1024;
@@ -2237,7 +2250,7 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
   if (bgk && cells >= 60000 && cells < 1500000) {
     return 512;
   }
-  return beyond_cache || (bgk && cells >= 1500000) ? 1024 : 0;
+  return beyond_cache || (bgk && cells >= 2400000) ? 1024 : 0;
 }
 
 // the lattice's second set of populations; false where it cannot be had: the
@@ -2334,7 +2347,10 @@ void launch_pair_mode(int mode, bool periodic, bool src_ring, bool dst_ring, dim
     case OLBGFX_FORCED_TRT:
       return launch_pair_form<S, NT, OLBGFX_FORCED_TRT, true>(src_ring, dst_ring, grid, stream, p);
     case OLBGFX_SMAGORINSKY_BGK:
-      return launch_pair_form<S, NT, OLBGFX_SMAGORINSKY_BGK, true>(src_ring, dst_ring, grid, stream, p);
+      if constexpr (sizeof(S) > 2) {
+        return launch_pair_form<S, NT, OLBGFX_SMAGORINSKY_BGK, true>(src_ring, dst_ring, grid, stream, p);
+      }
+      break;
     default:
       break;
     }
@@ -2442,7 +2458,8 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
       HIP_TRY(hipFree(L->stats_partial));
       L->stats_partial = nullptr;
     }
-    HIP_TRY(device_alloc(&L->stats_partial, 4 * sizeof(double) * (size_t)a.nblocks));
+    const uint32_t sums = (a.nblocks + kStatsChunk - 1) / kStatsChunk;
+    HIP_TRY(device_alloc(&L->stats_partial, 4 * sizeof(double) * ((size_t)a.nblocks + sums)));
     L->stats_capacity = a.nblocks;
     a.stats = L->stats_partial;
   }
@@ -2505,9 +2522,17 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
   }
   for (uint32_t k = first; k < steps; ++k) {
     for (int i = 0; i < Q; ++i) a.shift[i] = L->shift[i];
-    if (L->stats_on) {
+    // only the last step's statistics can be read
+    if (L->stats_on && k + 1 == steps) {
       launch_mode<S, true>(mode, grid, block, L->lds_reserve, stream, a);
-      stats_finalize<<<1, 256, 0, stream>>>(L->stats_partial, a.nblocks, L->stats_out);
+      const uint32_t sums = (a.nblocks + kStatsChunk - 1) / kStatsChunk;
+      if (sums == 1) {
+        stats_finalize<<<1, kStatsThreads, 0, stream>>>(L->stats_partial, a.nblocks, a.nblocks, L->stats_out);
+      } else {
+        double* second = L->stats_partial + 4 * (size_t)a.nblocks;
+        stats_finalize<<<sums, kStatsThreads, 0, stream>>>(L->stats_partial, a.nblocks, kStatsChunk, second);
+        stats_finalize<<<1, kStatsThreads, 0, stream>>>(second, sums, sums, L->stats_out);
+      }
     } else {
       launch_mode<S, false>(dominant, grid, block, L->lds_reserve, stream, a);
       if (split && L->residual_n > 0) {
@@ -2927,9 +2952,7 @@ olbgfx_status olbgfx_lattice_create(const olbgfx_lattice_desc* desc, olbgfx_latt
       device_alloc(&L->shift_dev, sizeof(L->shift)) != hipSuccess ||
       hipMemset(L->shift_dev, 0, sizeof(L->shift)) != hipSuccess ||
       device_alloc(&L->kinds_dev, sizeof(int32_t) * 256) != hipSuccess ||
-      hipMemset(L->kinds_dev, 0, sizeof(int32_t) * 256) != hipSuccess ||
-      device_alloc(&L->stats_out, 4 * sizeof(double)) != hipSuccess ||
-      hipMemset(L->stats_out, 0, 4 * sizeof(double)) != hipSuccess) {
+      hipMemset(L->kinds_dev, 0, sizeof(int32_t) * 256) != hipSuccess) {
     return cleanup(fail(OLBGFX_ERR_NOMEM, "device allocation failed"));
   }
   *out = L;
@@ -2960,7 +2983,9 @@ olbgfx_status olbgfx_lattice_destroy(olbgfx_lattice* L)
   hipFree(L->bzv_q);
   hipFree(L->bzv_v);
   hipFree(L->stats_partial);
-  hipFree(L->stats_out);
+  if (L->stats_out) {
+    (void)hipHostFree(L->stats_out);
+  }
   hipFree(L->residual_dev);
   drop_pair_buffer(L);
   for (hipEvent_t e : L->inflight_events) {
@@ -3430,6 +3455,16 @@ olbgfx_status olbgfx_set_statistics(olbgfx_lattice* L, int32_t on)
   if (check(L) != OLBGFX_OK) {
     return OLBGFX_ERR_INVALID;
   }
+  // the finalizing kernel writes its four sums to host memory: reading them
+  // after a step then takes the synchronisation alone, without a copy
+  if (on && !L->stats_out) {
+    if (hipHostMalloc((void**)&L->stats_out, 4 * sizeof(double), hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      L->stats_out = nullptr;
+      return fail(OLBGFX_ERR_NOMEM, "host allocation for the statistics failed");
+    }
+    std::fill(L->stats_out, L->stats_out + 4, 0.0);
+  }
   L->stats_on = on != 0;
   return OLBGFX_OK;
 }
@@ -3444,7 +3479,7 @@ olbgfx_status olbgfx_get_statistics(olbgfx_lattice* L, double out[4])
     return OLBGFX_OK;
   }
   HIP_TRY(hipDeviceSynchronize());
-  HIP_TRY(hipMemcpy(out, L->stats_out, 4 * sizeof(double), hipMemcpyDeviceToHost));
+  std::memcpy(out, L->stats_out, 4 * sizeof(double));
   return OLBGFX_OK;
 }
 
@@ -4594,8 +4629,10 @@ olbgfx_status save_state(olbgfx_lattice* L, hipStream_t stream, SavedState& out)
     return fail(OLBGFX_ERR_NOMEM, "not enough device memory to keep the lattice state while tuning");
   }
   HIP_TRY(hipMemcpyAsync(out.pop, L->pop, bytes, hipMemcpyDeviceToDevice, stream));
-  HIP_TRY(hipMemcpyAsync(out.stats, L->stats_out, sizeof(out.stats), hipMemcpyDeviceToHost, stream));
   HIP_TRY(hipStreamSynchronize(stream));
+  if (L->stats_out) {
+    std::memcpy(out.stats, L->stats_out, sizeof(out.stats));
+  }
   std::memcpy(out.shift, L->shift, sizeof(out.shift));
   out.stats_valid = L->stats_valid;
   return OLBGFX_OK;
@@ -4606,8 +4643,10 @@ olbgfx_status restore_state(const SavedState& s, hipStream_t stream)
   olbgfx_lattice* L = s.L;
   const size_t bytes = (size_t)Q * L->stride * L->elem;
   HIP_TRY(hipMemcpyAsync(L->pop, s.pop, bytes, hipMemcpyDeviceToDevice, stream));
-  HIP_TRY(hipMemcpyAsync(L->stats_out, s.stats, sizeof(s.stats), hipMemcpyHostToDevice, stream));
   HIP_TRY(hipStreamSynchronize(stream));
+  if (L->stats_out) {
+    std::memcpy(L->stats_out, s.stats, sizeof(s.stats));
+  }
   std::memcpy(L->shift, s.shift, sizeof(L->shift));
   L->stats_valid = s.stats_valid;
   return sync_shifts(L);

@@ -18,7 +18,7 @@ UNIFORM = [
     ("f32", BGK, (39, 41, 43), 3),       # 512 threads, one short row a tile
     ("f32", BGK, (20, 9, 513), 1),       # thin along y, long rows
     ("f32", BGK, (5, 700, 40), 2),
-    ("f32", BGK, (115, 131, 101), 1),    # 1024 threads
+    ("f32", BGK, (135, 139, 131), 1),    # 1024 threads
     ("f32", FORCED_TRT, (150, 163, 149), 2),
     ("f32", SMAGORINSKY_BGK, (161, 157, 141), 3),
     ("f16", BGK, (187, 190, 201), 1),
