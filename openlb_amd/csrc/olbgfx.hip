@@ -1068,7 +1068,7 @@ __device__ __forceinline__ void load_cell(const StepArgs<typename Storage<S>::A>
 
 // computeRho of cell m through its momenta
 template <typename S>
-__device__ typename Storage<S>::A momenta_rho(const StepArgs<typename Storage<S>::A>& a, uint32_t m)
+__device__ __forceinline__ typename Storage<S>::A momenta_rho(const StepArgs<typename Storage<S>::A>& a, uint32_t m)
 {
   using A = typename Storage<S>::A;
   A f[Q];
@@ -1111,7 +1111,7 @@ __device__ typename Storage<S>::A momenta_rho(const StepArgs<typename Storage<S>
 
 // computeU of cell m through its momenta
 template <typename S>
-__device__ void momenta_u(const StepArgs<typename Storage<S>::A>& a, uint32_t m, typename Storage<S>::A (&u)[3])
+__device__ __forceinline__ void momenta_u(const StepArgs<typename Storage<S>::A>& a, uint32_t m, typename Storage<S>::A (&u)[3])
 {
   using A = typename Storage<S>::A;
   const DynEntry<A>& e = a.table[a.mask[m]];
@@ -1156,22 +1156,6 @@ __device__ void momenta_u(const StepArgs<typename Storage<S>::A>& a, uint32_t m,
   }
 }
 
-// DirectedGradients3D along the boundary normal (finiteDifference3D.h:132-155):
-// -orient * (-3 u0 + 4 u1 - u2) / 2 with u1, u2 one and two cells inwards
-template <typename S>
-__device__ void one_sided(const StepArgs<typename Storage<S>::A>& a, uint32_t n, int64_t step, int orient,
-                          typename Storage<S>::A (&d)[3])
-{
-  using A = typename Storage<S>::A;
-  A u0[3], u1[3], u2[3];
-  momenta_u<S>(a, n, u0);
-  momenta_u<S>(a, (uint32_t)((int64_t)n - orient * step), u1);
-  momenta_u<S>(a, (uint32_t)((int64_t)n - 2 * orient * step), u2);
-  for (int b = 0; b < 3; ++b) {
-    d[b] = A(-orient) * ((-A(3) * u0[b] + A(4) * u1[b] - A(1) * u2[b]) / A(2));
-  }
-}
-
 // The cells whose momenta the edge or corner processor of cell n reads,
 // slot by slot.  Edge, plane p (the zero component of the normal), d1 and d2
 // the other axes with normal components n1 and n2: 0: n - n1 e_d1,
@@ -1201,82 +1185,134 @@ __device__ __forceinline__ uint32_t post_neighbor(uint32_t n, const int (&N)[3],
   return (uint32_t)((int64_t)n - m * N[k] * step[k]);
 }
 
-// One launch applies the processors of one list (edges, or corners: a
-// corner reads edge cells the edge processors rewrite, so the corners run in
-// a launch of their own after the edges).  A block takes 32 cells; lane
-// `slot` of a cell evaluates the momenta of one of its 7 neighbour cells
-// into LDS, so the ~13 neighbour evaluations of a cell run side by side
-// instead of one after another; lane 0 then combines them and writes the
-// cell's 19 populations, with the arithmetic of
-// OuterVelocityEdgeProcessor3D / OuterVelocityCornerProcessor3D
-// (boundary/boundaryPostProcessors3D.hh:164-294).
-constexpr uint32_t kPostCellsPerBlock = 32;
-
-template <typename S>
-__global__ void __launch_bounds__(256) k_velocity_post(const StepArgs<typename Storage<S>::A> a,
-                                                       const uint32_t* cells, uint32_t ncells)
+// What a processor computes from the momenta of its 7 slots (rho, u): the
+// density it imposes and the regularised non-equilibrium stress, with the
+// arithmetic of OuterVelocityEdgeProcessor3D / OuterVelocityCornerProcessor3D
+// (boundary/boundaryPostProcessors3D.hh:164-294)
+template <typename A>
+__device__ __forceinline__ void post_combine(const A (&mom)[8][4], const int (&N)[3], A omega, A& rho, A (&pi)[6])
 {
-  using A = typename Storage<S>::A;
-  __shared__ A mom[kPostCellsPerBlock][8][4];
-  const uint32_t local = threadIdx.x >> 3;
-  const int slot = (int)(threadIdx.x & 7u);
-  const uint32_t t = blockIdx.x * kPostCellsPerBlock + local;
-  const bool active = t < ncells;
-  const uint32_t n = active ? cells[t] : 0u;
-  const uint32_t code = active ? a.normal[n] : 13u;
-  const int N[3] = {normal_component(code, 0), normal_component(code, 1), normal_component(code, 2)};
-  const int64_t step[3] = {(int64_t)a.py * a.pz, (int64_t)a.pz, 1};
-  if (active && slot < kPostSlots) {
-    const uint32_t m = post_neighbor(n, N, step, slot);
-    A u[3];
-    momenta_u<S>(a, m, u);
-    mom[local][slot][0] = momenta_rho<S>(a, m);
-    mom[local][slot][1] = u[0];
-    mom[local][slot][2] = u[1];
-    mom[local][slot][3] = u[2];
-  }
-  __syncthreads();
-  if (!active || slot != 0) {
-    return;
-  }
-  const DynEntry<A>& e = a.table[a.mask[n]];
   // DirectedGradients3D along a normal (finiteDifference3D.h:132-155):
   // -orient * (-3 u0 + 4 u1 - u2) / 2 with u1, u2 one and two cells inwards
   auto one_sided = [&](int s1, int s2, int orient, A (&d)[3]) {
     for (int b = 0; b < 3; ++b) {
-      d[b] = A(-orient) * ((-A(3) * mom[local][6][1 + b] + A(4) * mom[local][s1][1 + b] -
-                            A(1) * mom[local][s2][1 + b]) / A(2));
+      d[b] = A(-orient) * ((-A(3) * mom[6][1 + b] + A(4) * mom[s1][1 + b] - A(1) * mom[s2][1 + b]) / A(2));
     }
   };
-  A rho;
   A du[3][3];
   if (N[0] == 0 || N[1] == 0 || N[2] == 0) {
     // OuterVelocityEdgeProcessor3D<plane, normal1, normal2>
     const int p = N[0] == 0 ? 0 : (N[1] == 0 ? 1 : 2);
     const int d1 = (p + 1) % 3, d2 = (p + 2) % 3;
-    const A rho10 = mom[local][0][0], rho01 = mom[local][1][0];
-    const A rho20 = mom[local][2][0], rho02 = mom[local][3][0];
+    const A rho10 = mom[0][0], rho01 = mom[1][0];
+    const A rho20 = mom[2][0], rho02 = mom[3][0];
     rho = A(2) / A(3) * (rho01 + rho10) - A(1) / A(6) * (rho02 + rho20);
-    for (int b = 0; b < 3; ++b) du[p][b] = (mom[local][4][1 + b] - mom[local][5][1 + b]) / A(2);
+    for (int b = 0; b < 3; ++b) du[p][b] = (mom[4][1 + b] - mom[5][1 + b]) / A(2);
     one_sided(0, 2, N[d1], du[d1]);
     one_sided(1, 3, N[d2], du[d2]);
   } else {
     // OuterVelocityCornerProcessor3D<xNormal, yNormal, zNormal>
-    const A rho100 = mom[local][0][0], rho010 = mom[local][1][0], rho001 = mom[local][2][0];
-    const A rho200 = mom[local][3][0], rho020 = mom[local][4][0], rho002 = mom[local][5][0];
+    const A rho100 = mom[0][0], rho010 = mom[1][0], rho001 = mom[2][0];
+    const A rho200 = mom[3][0], rho020 = mom[4][0], rho002 = mom[5][0];
     rho = A(4) / A(9) * (rho001 + rho010 + rho100) - A(1) / A(9) * (rho002 + rho020 + rho200);
     for (int ax = 0; ax < 3; ++ax) one_sided(ax, 3 + ax, N[ax], du[ax]);
   }
   // regularised populations (boundaryPostProcessors3D.hh:196-215)
-  const A s_to_pi = -rho / A(3) / e.omega;
-  const A pi[6] = {A(2) * du[0][0] * s_to_pi, (du[0][1] + du[1][0]) * s_to_pi, (du[0][2] + du[2][0]) * s_to_pi,
-                   A(2) * du[1][1] * s_to_pi, (du[1][2] + du[2][1]) * s_to_pi, A(2) * du[2][2] * s_to_pi};
+  const A s_to_pi = -rho / A(3) / omega;
+  pi[0] = A(2) * du[0][0] * s_to_pi;
+  pi[1] = (du[0][1] + du[1][0]) * s_to_pi;
+  pi[2] = (du[0][2] + du[2][0]) * s_to_pi;
+  pi[3] = A(2) * du[1][1] * s_to_pi;
+  pi[4] = (du[1][2] + du[2][1]) * s_to_pi;
+  pi[5] = A(2) * du[2][2] * s_to_pi;
+}
+
+// The processors of the listed cells, edges before corners in one launch or in
+// two.  A wave takes 8 cells, 8 lanes each: lane `slot` of a cell evaluates the
+// momenta of one of its 7 neighbour cells into LDS (the density only of the
+// slots whose density is used), so the neighbour evaluations of a cell run side
+// by side; lane 0 then combines them and writes the cell's 19 populations.
+// The chain of dependent loads (cell, normal, id, table, populations) bounds
+// it.  On the 1200 edges and 8 corners of a 101^3 cavity in FP32 a launch each
+// of four-wave workgroups, which held 38 CUs, took 13.2 + 5.2 us; workgroups of
+// one wave, densities only where used and one launch for both take 9.5 us.
+//
+// A corner reads the density of edge cells that the edge processors rewrite.
+// In the joint launch (CORNERS) each corner has a wave of its own that forms
+// the rewritten populations of those up to 6 edge cells again, rounded as they
+// are stored, and sums them: the density that a later launch would read.  Its
+// group `local` < 7 of 8 lanes stands for slot `local` of the corner, cell m:
+// lanes 0-6 for the slots of m's own processor, lane 7 for m itself.  The host
+// makes sure that no edge reads the density of a corner.
+template <typename S, bool CORNERS>
+__global__ void __launch_bounds__(64) k_velocity_post(const StepArgs<typename Storage<S>::A> a, const uint32_t* cells,
+                                                      uint32_t ncells, uint32_t nedges)
+{
+  using A = typename Storage<S>::A;
+  using St = Storage<S>;
+  __shared__ A mom[8][8][4];
+  const uint32_t local = threadIdx.x >> 3;
+  const int slot = (int)(threadIdx.x & 7u);
+  const int64_t step[3] = {(int64_t)a.py * a.pz, (int64_t)a.pz, 1};
+  const uint32_t edge_waves = (nedges + 7) / 8;
+  const bool corner_wave = CORNERS && blockIdx.x >= edge_waves;  // uniform
+  const uint32_t t = corner_wave ? nedges + blockIdx.x - edge_waves : blockIdx.x * 8 + local;
+  const bool listed = corner_wave || t < (CORNERS ? nedges : ncells);
+  const uint32_t n = listed ? cells[t] : 0u;
+  const uint32_t code = listed ? a.normal[n] : 13u;
+  const int N[3] = {normal_component(code, 0), normal_component(code, 1), normal_component(code, 2)};
+  // the cell whose processor this group evaluates, and its normal
+  uint32_t m = n;
+  int M[3] = {N[0], N[1], N[2]};
+  bool rewritten = false;
+  if (corner_wave) {
+    m = post_neighbor(n, N, step, (int)min(local, 6u));
+    const uint32_t mcode = a.normal[m];
+    for (int ax = 0; ax < 3; ++ax) M[ax] = normal_component(mcode, ax);
+    rewritten = local < 6 && a.table[a.mask[m]].kind == OLBGFX_FIXED_VELOCITY &&
+                (M[0] != 0) + (M[1] != 0) + (M[2] != 0) == 2;
+  }
+  const bool edge = M[0] == 0 || M[1] == 0 || M[2] == 0;
+  const bool itself = corner_wave && slot == kPostSlots;
+  if (corner_wave ? (itself ? local < 7 : rewritten) : listed && slot < kPostSlots) {
+    const uint32_t at = itself ? m : post_neighbor(m, M, step, slot);
+    A u[3];
+    momenta_u<S>(a, at, u);
+    const bool density = itself ? local < 6 && !rewritten : slot < (edge ? 4 : 6);
+    mom[local][slot][0] = density ? momenta_rho<S>(a, at) : A(0);
+    for (int b = 0; b < 3; ++b) mom[local][slot][1 + b] = u[b];
+  }
+  __syncthreads();
+  A rho, pi[6];
+  if (corner_wave) {
+    // the groups' results side by side in group 7, which has none of its own
+    if (slot == 0 && local < 7) {
+      A r = mom[local][7][0];
+      if (rewritten) {
+        post_combine(mom[local], M, a.table[a.mask[m]].omega, rho, pi);
+        const A u[3] = {mom[local][7][1], mom[local][7][2], mom[local][7][3]};
+        const A usqr = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+        A s = A(0);
+#pragma unroll
+        for (int i = 0; i < Q; ++i) s += St::unpack(St::pack(feq_i(i, rho, u, usqr) + pi_to_fneq(i, pi)));
+        r = s + A(1);
+      }
+      mom[7][local][0] = r;
+      for (int b = 1; b < 4; ++b) mom[7][local][b] = mom[local][7][b];
+    }
+    __syncthreads();
+  }
+  if (!listed || slot != 0 || (corner_wave && local != 0)) {
+    return;
+  }
+  post_combine(mom[corner_wave ? 7 : local], N, a.table[a.mask[n]].omega, rho, pi);
+  const DynEntry<A>& e = a.table[a.mask[n]];
   const A u[3] = {wall_component(a, e, n, 0), wall_component(a, e, n, 1), wall_component(a, e, n, 2)};
   const A usqr = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
     *ring_at<S>(a.pop, a.stride, i, ring_slot(n, a.shift[i], a.count)) =
-        Storage<S>::pack(feq_i(i, rho, u, usqr) + pi_to_fneq(i, pi));
+        St::pack(feq_i(i, rho, u, usqr) + pi_to_fneq(i, pi));
   }
 }
 
@@ -1288,32 +1324,62 @@ __global__ void __launch_bounds__(256) k_velocity_post(const StepArgs<typename S
 // to the regularised value feq(rho, u) + fneq(Pi(grad u)).  The new
 // populations go to `out` (19 per listed cell) and k_plane_fd_store writes
 // them back, so no processor reads a value another one has rewritten.
+//
+// As in k_velocity_post, a wave takes 8 cells and lane `slot` of a cell one of
+// the 7 cells its gradients read: 0 itself, 1 and 2 inwards, 3 to 6 its
+// neighbours along the wall.  On the 2 x 39 x 39 faces of a channel in FP64 one
+// thread a cell, 209 VGPRs and 12 workgroups in all, took 18.9 us and its store
+// 6.4; now 9.6 and 3.1 us.
 template <typename S>
-__global__ void __launch_bounds__(256) k_plane_fd(const StepArgs<typename Storage<S>::A> a, const uint32_t* cells,
-                                                  uint32_t ncells, typename Storage<S>::A* out)
+__global__ void __launch_bounds__(64) k_plane_fd(const StepArgs<typename Storage<S>::A> a, const uint32_t* cells,
+                                                 uint32_t ncells, typename Storage<S>::A* out)
 {
   using A = typename Storage<S>::A;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ncells) {
+  __shared__ A mom[8][8][4];
+  const uint32_t local = threadIdx.x >> 3;
+  const int slot = (int)(threadIdx.x & 7u);
+  const uint32_t t = blockIdx.x * 8 + local;
+  const bool active = t < ncells;
+  const uint32_t n = active ? cells[t] : 0u;
+  int dir = 0, orient = 0;
+  if (active) {
+    flat_normal(a.normal[n], dir, orient);
+  }
+  const int64_t step[3] = {(int64_t)a.py * a.pz, (int64_t)a.pz, 1};
+  const int w1 = dir == 0 ? 1 : 0, w2 = dir == 2 ? 1 : 2;  // the axes along the wall, ascending
+  if (active && slot < 7) {
+    int64_t d;
+    switch (slot) {
+    case 0: d = 0; break;
+    case 1: d = -orient * step[dir]; break;
+    case 2: d = -2 * orient * step[dir]; break;
+    case 3: d = step[w1]; break;
+    case 4: d = -step[w1]; break;
+    case 5: d = step[w2]; break;
+    default: d = -step[w2]; break;
+    }
+    const uint32_t m = (uint32_t)((int64_t)n + d);
+    A u[3];
+    momenta_u<S>(a, m, u);
+    mom[local][slot][0] = slot == 0 ? momenta_rho<S>(a, m) : A(0);
+    for (int b = 0; b < 3; ++b) mom[local][slot][1 + b] = u[b];
+  }
+  __syncthreads();
+  if (!active || slot != 0) {
     return;
   }
-  const uint32_t n = cells[t];
-  int dir, orient;
-  flat_normal(a.normal[n], dir, orient);
-  const int64_t step[3] = {(int64_t)a.py * a.pz, (int64_t)a.pz, 1};
   const DynEntry<A>& e = a.table[a.mask[n]];
-  const A rho = momenta_rho<S>(a, n);
-  A u[3];
-  momenta_u<S>(a, n, u);
+  const A rho = mom[local][0][0];
+  const A u[3] = {mom[local][0][1], mom[local][0][2], mom[local][0][3]};
   A du[3][3];
   for (int d = 0; d < 3; ++d) {
-    if (d == dir) {
-      one_sided<S>(a, n, step[d], orient, du[d]);
-    } else {
-      A up[3], um[3];
-      momenta_u<S>(a, (uint32_t)((int64_t)n + step[d]), up);
-      momenta_u<S>(a, (uint32_t)((int64_t)n - step[d]), um);
-      for (int b = 0; b < 3; ++b) du[d][b] = (up[b] - um[b]) / A(2);
+    for (int b = 0; b < 3; ++b) {
+      if (d == dir) {
+        du[d][b] = A(-orient) * ((-A(3) * u[b] + A(4) * mom[local][1][1 + b] - A(1) * mom[local][2][1 + b]) / A(2));
+      } else {
+        const int s = d == w1 ? 3 : 5;
+        du[d][b] = (mom[local][s][1 + b] - mom[local][s + 1][1 + b]) / A(2);
+      }
     }
   }
   const A s_to_pi = -rho / A(3) / e.omega;
@@ -1326,6 +1392,7 @@ __global__ void __launch_bounds__(256) k_plane_fd(const StepArgs<typename Storag
   }
 }
 
+// one thread a population, population blockIdx.y
 template <typename S>
 __global__ void __launch_bounds__(256) k_plane_fd_store(const StepArgs<typename Storage<S>::A> a,
                                                         const uint32_t* cells, uint32_t ncells,
@@ -1335,11 +1402,9 @@ __global__ void __launch_bounds__(256) k_plane_fd_store(const StepArgs<typename 
   if (t >= ncells) {
     return;
   }
-  const uint32_t n = cells[t];
-#pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    *ring_at<S>(a.pop, a.stride, i, ring_slot(n, a.shift[i], a.count)) = Storage<S>::pack(out[(size_t)i * ncells + t]);
-  }
+  const int i = (int)blockIdx.y;
+  *ring_at<S>(a.pop, a.stride, i, ring_slot(cells[t], a.shift[i], a.count)) =
+      Storage<S>::pack(out[(size_t)i * ncells + t]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1867,6 +1932,7 @@ struct olbgfx_lattice {
   uint8_t* normal_dev = nullptr;     // code 9(nx+1)+3(ny+1)+(nz+1) per cell
   uint32_t* post_dev = nullptr;
   uint32_t post_edges = 0, post_corners = 0;
+  bool post_joint = false;           // edges and corners in one launch
   uint32_t* fd_dev = nullptr;        // flat interpolated cells (PlaneFdBoundaryProcessor3D)
   void* fd_out = nullptr;            // their new populations, 19 per cell in the arithmetic type
   uint32_t fd_n = 0;
@@ -2100,20 +2166,27 @@ olbgfx_status launch_post(olbgfx_lattice* L, StepArgs<typename Storage<S>::A>& a
                                                             (const A*)L->bzv_v, L->bzv_n);
     HIP_TRY(hipGetLastError());
   }
-  if (L->post_edges) {
-    k_velocity_post<S><<<(L->post_edges + kPostCellsPerBlock - 1) / kPostCellsPerBlock, 256, 0, stream>>>(
-        a, L->post_dev, L->post_edges);
+  const uint32_t edge_waves = (L->post_edges + 7) / 8;
+  if (L->post_joint && L->post_edges && L->post_corners) {
+    k_velocity_post<S, true><<<edge_waves + L->post_corners, 64, 0, stream>>>(
+        a, L->post_dev, L->post_edges + L->post_corners, L->post_edges);
     HIP_TRY(hipGetLastError());
-  }
-  if (L->post_corners) {
-    k_velocity_post<S><<<(L->post_corners + kPostCellsPerBlock - 1) / kPostCellsPerBlock, 256, 0, stream>>>(
-        a, L->post_dev + L->post_edges, L->post_corners);
-    HIP_TRY(hipGetLastError());
+  } else {
+    if (L->post_edges) {
+      k_velocity_post<S, false><<<edge_waves, 64, 0, stream>>>(a, L->post_dev, L->post_edges, 0);
+      HIP_TRY(hipGetLastError());
+    }
+    if (L->post_corners) {
+      k_velocity_post<S, false><<<(L->post_corners + 7) / 8, 64, 0, stream>>>(a, L->post_dev + L->post_edges,
+                                                                             L->post_corners, 0);
+      HIP_TRY(hipGetLastError());
+    }
   }
   if (L->fd_n) {
-    k_plane_fd<S><<<(L->fd_n + 255) / 256, 256, 0, stream>>>(a, L->fd_dev, L->fd_n, (A*)L->fd_out);
+    k_plane_fd<S><<<(L->fd_n + 7) / 8, 64, 0, stream>>>(a, L->fd_dev, L->fd_n, (A*)L->fd_out);
     HIP_TRY(hipGetLastError());
-    k_plane_fd_store<S><<<(L->fd_n + 255) / 256, 256, 0, stream>>>(a, L->fd_dev, L->fd_n, (const A*)L->fd_out);
+    k_plane_fd_store<S><<<dim3((L->fd_n + 255) / 256, Q), 256, 0, stream>>>(a, L->fd_dev, L->fd_n,
+                                                                          (const A*)L->fd_out);
     HIP_TRY(hipGetLastError());
   }
   return OLBGFX_OK;
@@ -2777,6 +2850,7 @@ olbgfx_status prepare_boundary(olbgfx_lattice* L)
     for (uint32_t n : edges) in[n] = 1;
     for (uint32_t n : corners) in[n] = 2;
     const int64_t step[3] = {(int64_t)L->py * L->pz, (int64_t)L->pz, 1};
+    L->post_joint = true;
     for (int list = 1; list <= 2; ++list) {
       for (uint32_t n : (list == 1 ? edges : corners)) {
         int N[3];
@@ -2785,6 +2859,14 @@ olbgfx_status prepare_boundary(olbgfx_lattice* L)
           if (N[ax] == 0) continue;
           for (int k = 1; k <= 2; ++k) {
             const int64_t m = (int64_t)n - (int64_t)k * N[ax] * step[ax];
+            // not in one launch: edges that read a corner's density, and
+            // corners that read an edge of the padding (no processor runs there)
+            const int8_t* nm = &L->host_normals[3 * (size_t)m];
+            const bool edge_cell = L->table[L->host_mask[(size_t)m]].kind == OLBGFX_FIXED_VELOCITY &&
+                                   (nm[0] != 0) + (nm[1] != 0) + (nm[2] != 0) == 2;
+            if (list == 1 ? in[(size_t)m] == 2 : edge_cell && in[(size_t)m] != 1) {
+              L->post_joint = false;
+            }
             if (in[(size_t)m] == list) {
               return fail(OLBGFX_ERR_UNSUPPORTED,
                           "a LocalVelocity edge or corner processor reads the density of another one of its kind");
