@@ -302,15 +302,17 @@ olbgfx_status olbgfx_compute_rho_u(olbgfx_lattice* lattice, int32_t value_type, 
 /* ---- launch configuration ---------------------------------------------------
  * threads per block of the step kernel (64..256, multiple of 64; 0 = 256) and
  * an occupancy cap in waves per SIMD (1..8; 0 = as many as registers allow),
- * enforced by reserving LDS per block.  Used by the autotuner; no reference
+ * enforced by reserving LDS per block.  Until this is called, 256 threads and
+ * a cap chosen by the size of the lattice.  Used by the autotuner; no reference
  * counterpart (the reference fixes 64-thread blocks,
  * core/platform/gpu/hip/operator.hh:426-433). */
 olbgfx_status olbgfx_set_launch(olbgfx_lattice* lattice, uint32_t block_threads,
                                 uint32_t waves_per_simd);
 
-/* order in which the step kernel's blocks visit the cells: -1 (default) gives
- * each of the 8 XCDs one contiguous part of the block; k in [0, 12] lets the
- * XCDs take turns on runs of 2^k consecutive blocks.  Results do not depend
+/* order in which the step kernel's blocks visit the cells: -1 gives each of the
+ * 8 XCDs one contiguous part of the block; k in [0, 12] lets the XCDs take
+ * turns on runs of 2^k consecutive blocks.  Until this is called, chosen by the
+ * size of the lattice.  Results do not depend
  * on it.  Used by the autotuner; no reference counterpart. */
 olbgfx_status olbgfx_set_block_order(olbgfx_lattice* lattice, int32_t xcd_run_log2);
 

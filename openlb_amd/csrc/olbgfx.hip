@@ -1922,10 +1922,10 @@ struct olbgfx_lattice {
   bool stats_on = false;
   bool stats_valid = false;
   int32_t uniform_id = 0;     // all cells start with id 0 = NoDynamics
-  uint32_t core_ids = 1;      // bit k: some core cell has id k
   uint32_t block_threads = 256;
   uint32_t lds_reserve = 0;    // dynamic LDS per block that limits occupancy
   int32_t xcd_run_log2 = -1;   // block order of the step kernel (olbgfx_set_block_order)
+  bool launch_given = false, order_given = false;  // else chosen by size (default_launch)
   // LocalVelocity boundaries: discrete normals, and the cells whose
   // post-processors run after each step (edges first, then corners)
   std::vector<int8_t> host_normals;  // 3 per cell, empty = none
@@ -1975,6 +1975,8 @@ struct olbgfx_lattice {
   void* pair_pop = nullptr;
   int pair_device = 0;
   PairPlan pair_plan;
+  bool walls_only = false;           // wall_mode, as of wall_version
+  uint64_t wall_version = ~0ull;
   bool pair_enabled = true;          // off while the tuner times single steps
 };
 
@@ -2045,6 +2047,47 @@ void fill_table(const olbgfx_lattice* L, DynEntry<A>* t)
   }
 }
 
+// LDS to reserve per block of block_threads so that at most waves_per_simd
+// waves share a SIMD (0: no cap)
+uint32_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
+{
+  if (waves_per_simd == 0) {
+    return 0;
+  }
+  // a CU has 4 SIMDs and 160 KiB of LDS: reserving LDS per block caps the
+  // blocks that fit on one CU, and with them the waves per SIMD
+  const uint32_t waves_per_block = block_threads / 64;
+  const uint32_t blocks_per_cu = std::max(1u, 4 * waves_per_simd / waves_per_block);
+  uint32_t lds = kLdsPerCu / blocks_per_cu / 1024 * 1024;
+  if (lds * (blocks_per_cu + 1) <= kLdsPerCu) {
+    lds += 1024;
+  }
+  return std::min(lds, kLdsPerCu - 4096);  // room for the kernel's own reduction scratch
+}
+
+// Occupancy cap and block order of single steps until they are set by a call.
+// Where the populations exceed the Infinity Cache the open DRAM pages decide:
+// fewer waves in flight (4-byte storage) and XCDs taking turns on short runs
+// keep the cells in flight together.  us a step, no cap and contiguous parts
+// against these: 512^3 FP32 4350 / 3960, FP16 2228 / 2076; slab 64x512x512 FP32
+// 538 / 497, FP16 279 / 263; 256^3 FP32 550 / 509, cavity 552 / 509, FP64 1051
+// / 1018; porous channel FP16 125 / 120.  Between 256 MiB and 1 GiB contiguous
+// parts stay better in 4-byte storage (40x300x400 capped: 138 against 144, 150
+// without the cap), and below 224 MiB the cache serves them best (160^3 FP16
+// 47 against 49, cavity 33^3 FP32 4.8 against 5.3).
+void default_launch(const olbgfx_lattice* L, uint32_t& lds, int32_t& order)
+{
+  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
+  lds = L->launch_given ? L->lds_reserve : (L->elem == 4 && mib >= 256 ? lds_for(L->block_threads, 4) : 0);
+  if (L->order_given) {
+    order = L->xcd_run_log2;
+  } else if (L->elem == 2) {
+    order = mib >= 224 ? 3 : -1;
+  } else {
+    order = mib >= 1024 ? 4 : -1;
+  }
+}
+
 template <typename A>
 olbgfx_status fill_args(olbgfx_lattice* L, StepArgs<A>& a, bool device_shifts)
 {
@@ -2069,7 +2112,8 @@ olbgfx_status fill_args(olbgfx_lattice* L, StepArgs<A>& a, bool device_shifts)
   a.ncore = (uint32_t)D.nx * a.nyz;
   a.nblocks = (a.ncore + L->block_threads - 1) / L->block_threads;
   a.blocks_per_xcd = (a.nblocks + 7) / 8;
-  a.xcd_run_log2 = L->xcd_run_log2;
+  uint32_t lds = 0;
+  default_launch(L, lds, a.xcd_run_log2);
   if (a.xcd_run_log2 >= 0) {
     const uint32_t run = 1u << a.xcd_run_log2;
     a.blocks_per_xcd = (a.blocks_per_xcd + run - 1) / run * run;
@@ -2497,21 +2541,26 @@ olbgfx_status launch_pair(olbgfx_lattice* L, const StepArgs<typename Storage<S>:
   return OLBGFX_OK;
 }
 
-// kWithWalls + BGK where the core cells hold no other kind besides bounce-back
+// kWithWalls + BGK where the mask holds no other kind besides bounce-back
 // and NoDynamics, -1 otherwise.  That kernel has one bulk kind and its
 // parameters in scalar registers (us a step, against the kernel of every kind:
 // cavity 160^3 FP32 94 / 99, 256^3 387 / 404, 160^3 FP64 180 / 199); the same
 // for ForcedTRT was slower (porous channel FP32 154 / 149, 160^3 FP64 223 / 207).
-int wall_mode(const olbgfx_lattice* L)
+int wall_mode(olbgfx_lattice* L)
 {
-  for (int id = 0; id < OLBGFX_MAX_DYNAMICS; ++id) {
-    const int k = L->table[id].kind;
-    if ((L->core_ids >> id & 1) && k != OLBGFX_BGK && k != OLBGFX_NO_DYNAMICS && k != OLBGFX_BOUNCE_BACK &&
-        k != OLBGFX_BOUNCE_BACK_VELOCITY) {
-      return -1;
+  if (L->wall_version != L->version) {
+    L->wall_version = L->version;
+    L->walls_only = true;
+    for (int id = 0; id < OLBGFX_MAX_DYNAMICS && L->walls_only; ++id) {
+      const int k = L->table[id].kind;
+      // other kinds must not occur, in the padding either (found at once where
+      // they do)
+      L->walls_only = k == OLBGFX_BGK || k == OLBGFX_NO_DYNAMICS || k == OLBGFX_BOUNCE_BACK ||
+                      k == OLBGFX_BOUNCE_BACK_VELOCITY ||
+                      std::memchr(L->host_mask.data(), id, L->host_mask.size()) == nullptr;
     }
   }
-  return kWithWalls + OLBGFX_BGK;
+  return L->walls_only ? kWithWalls + OLBGFX_BGK : -1;
 }
 
 template <typename S>
@@ -2538,6 +2587,9 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
   }
   const dim3 grid(8 * a.blocks_per_xcd);
   const dim3 block(L->block_threads);
+  uint32_t lds = 0;
+  int32_t order = -1;
+  default_launch(L, lds, order);
   int mode = L->uniform_id >= 0 ? L->table[L->uniform_id].kind : -1;
   if (L->boundary_kinds) {
     mode = kMaskedBoundary;
@@ -2597,7 +2649,7 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
     for (int i = 0; i < Q; ++i) a.shift[i] = L->shift[i];
     // only the last step's statistics can be read
     if (L->stats_on && k + 1 == steps) {
-      launch_mode<S, true>(mode, grid, block, L->lds_reserve, stream, a);
+      launch_mode<S, true>(mode, grid, block, lds, stream, a);
       const uint32_t sums = (a.nblocks + kStatsChunk - 1) / kStatsChunk;
       if (sums == 1) {
         stats_finalize<<<1, kStatsThreads, 0, stream>>>(L->stats_partial, a.nblocks, a.nblocks, L->stats_out);
@@ -2607,7 +2659,7 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
         stats_finalize<<<1, kStatsThreads, 0, stream>>>(second, sums, sums, L->stats_out);
       }
     } else {
-      launch_mode<S, false>(dominant, grid, block, L->lds_reserve, stream, a);
+      launch_mode<S, false>(dominant, grid, block, lds, stream, a);
       if (split && L->residual_n > 0) {
         for (int i = 0; i < Q; ++i) rest.shift[i] = L->shift[i];
         const dim3 rgrid((L->residual_n + 255) / 256);
@@ -2746,21 +2798,25 @@ olbgfx_status check(const olbgfx_lattice* L)
   return OLBGFX_OK;
 }
 
-// the ids of the core cells, and the id they share if they do
 void recompute_uniform(olbgfx_lattice* L)
 {
   const olbgfx_lattice_desc& D = L->desc;
-  uint32_t ids = 0;
-  for (int x = 0; x < D.nx; ++x) {
-    for (int y = 0; y < D.ny; ++y) {
+  int id = -2;
+  for (int x = 0; x < D.nx && id != -1; ++x) {
+    for (int y = 0; y < D.ny && id != -1; ++y) {
       const size_t base = ((size_t)(x + D.padding) * L->py + (y + D.padding)) * L->pz + D.padding;
       for (int z = 0; z < D.nz; ++z) {
-        ids |= 1u << L->host_mask[base + z];
+        const int v = L->host_mask[base + z];
+        if (id == -2) {
+          id = v;
+        } else if (v != id) {
+          id = -1;
+          break;
+        }
       }
     }
   }
-  L->core_ids = ids;
-  L->uniform_id = (ids & (ids - 1)) == 0 ? __builtin_ctz(ids) : -1;
+  L->uniform_id = id < 0 ? -1 : id;
 }
 
 // find the LocalVelocity cells and the post-processed edges and corners;
@@ -3722,20 +3778,9 @@ olbgfx_status olbgfx_set_launch(olbgfx_lattice* L, uint32_t block_threads, uint3
   if (waves_per_simd > 8) {
     return fail(OLBGFX_ERR_INVALID, "waves per SIMD must be in [0, 8]");
   }
-  uint32_t lds = 0;
-  if (waves_per_simd > 0) {
-    // a CU has 4 SIMDs and 160 KiB of LDS: reserving LDS per block caps the
-    // blocks that fit on one CU, and with them the waves per SIMD
-    const uint32_t waves_per_block = block_threads / 64;
-    const uint32_t blocks_per_cu = std::max(1u, 4 * waves_per_simd / waves_per_block);
-    lds = kLdsPerCu / blocks_per_cu / 1024 * 1024;
-    if (lds * (blocks_per_cu + 1) <= kLdsPerCu) {
-      lds += 1024;
-    }
-    lds = std::min(lds, kLdsPerCu - 4096);  // room for the kernel's own reduction scratch
-  }
   L->block_threads = block_threads;
-  L->lds_reserve = lds;
+  L->lds_reserve = lds_for(block_threads, waves_per_simd);
+  L->launch_given = true;
   return OLBGFX_OK;
 }
 
@@ -3748,6 +3793,7 @@ olbgfx_status olbgfx_set_block_order(olbgfx_lattice* L, int32_t xcd_run_log2)
     return fail(OLBGFX_ERR_INVALID, "block order must be -1 or a run length 2^k with k in [0, 12]");
   }
   L->xcd_run_log2 = xcd_run_log2;
+  L->order_given = true;
   return OLBGFX_OK;
 }
 
@@ -3801,20 +3847,6 @@ struct olbgfx_ensemble {
 };
 
 namespace {
-
-size_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
-{
-  if (waves_per_simd == 0) {
-    return 0;
-  }
-  const uint32_t waves_per_block = block_threads / 64;
-  const uint32_t blocks_per_cu = std::max(1u, 4 * waves_per_simd / waves_per_block);
-  uint32_t lds = kLdsPerCu / blocks_per_cu / 1024 * 1024;
-  if (lds * (blocks_per_cu + 1) <= kLdsPerCu) {
-    lds += 1024;
-  }
-  return std::min(lds, kLdsPerCu - 4096);
-}
 
 // host mirror of the offsets after `steps` more steps
 void advance_host_shifts(olbgfx_lattice* L, uint64_t steps)
