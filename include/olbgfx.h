@@ -338,7 +338,9 @@ olbgfx_status olbgfx_ensemble_set_launch(olbgfx_ensemble* ensemble, uint32_t blo
  * each group advances steps_per_group steps (1..1024) before the next group
  * runs; members are independent, so every member still ends a call
  * `steps` steps further.  A group that fits the 256 MB Infinity Cache is then
- * re-read from it.  ticket = 1 lets the last block of each launch advance the
+ * re-read from it.  Until this is called, groups of 200 MiB advance all steps
+ * of a call, and calls of fewer than 4 steps run all members in one launch.
+ * ticket = 1 lets the last block of each launch advance the
  * ring offsets (one launch per group step); 0 uses a separate small kernel.
  * Drops a captured graph.  Used by the autotuner. */
 olbgfx_status olbgfx_ensemble_set_schedule(olbgfx_ensemble* ensemble, uint64_t group_bytes,

@@ -3811,6 +3811,15 @@ olbgfx_status olbgfx_synchronize(olbgfx_lattice* L)
 // ---------------------------------------------------------------------------
 // ensemble of independent lattices
 
+// Default schedule.  64 cavities of 32 to 128 cells a side, us an ensemble step
+// in calls of 20 steps: all members a launch FP32 1630, FP16 913; groups of 160,
+// 180, 208 and 240 MiB FP32 1259, 1238, 1231, 1257, FP16 744, 725, 716, 814
+// (smaller groups leave CUs idle, larger ones fall out of the cache).  A group
+// has to come back to its rings a few times: groups of 208 MiB with 1, 2 and 4
+// steps each take FP32 1673, 1479, 1358, FP16 978, 947, 858.
+constexpr uint64_t kGroupBytes = 200ull << 20;
+constexpr uint32_t kGroupSteps = 4;
+
 struct olbgfx_ensemble {
   std::vector<olbgfx_lattice*> members;
   int32_t storage = OLBGFX_STORE_F32;
@@ -3831,9 +3840,12 @@ struct olbgfx_ensemble {
   // schedule: members are packed into groups of at most group_bytes of
   // population storage (0 = one group), and each group advances
   // steps_per_group steps before the next group runs, so a group that fits
-  // the 256 MB Infinity Cache is re-read from it instead of from HBM
-  uint64_t group_bytes = 0;
+  // the 256 MB Infinity Cache is re-read from it instead of from HBM.
+  // Until olbgfx_ensemble_set_schedule: kGroupBytes and all steps of a call,
+  // or one launch over all groups for calls of fewer than kGroupSteps steps
+  uint64_t group_bytes = kGroupBytes;
   uint32_t steps_per_group = 1;
+  bool schedule_given = false, launch_given = false;
   uint32_t ticket = 0;               // 1: last block advances the offsets; 0: separate kernel
   uint64_t grouped_bytes = ~0ull;
   std::vector<uint32_t> order;       // member index of each descriptor slot
@@ -3979,10 +3991,29 @@ template <typename S>
 olbgfx_status ensemble_enqueue(olbgfx_ensemble* E, uint32_t steps, hipStream_t stream)
 {
   using A = typename Storage<S>::A;
+  std::vector<GroupArgs> groups = E->groups;
+  uint32_t per_group = E->steps_per_group;
+  size_t lds = E->lds;
+  if (!E->schedule_given) {
+    per_group = 1024;
+    if (steps < kGroupSteps) {
+      // the tiles and members of all groups lie one after another
+      GroupArgs all = groups.front();
+      all.ntiles = E->ntiles;
+      all.member_end = groups.back().member_end;
+      groups.assign(1, all);
+      per_group = 1;
+      if (!E->launch_given) {
+        // as in default_launch: all members FP32 1630 / 1552 us with 4 waves a
+        // SIMD, FP16 913 / 891 with 5
+        lds = lds_for(E->block_threads, sizeof(S) == 4 ? 4 : (sizeof(S) == 2 ? 5 : 0));
+      }
+    }
+  }
   uint32_t done = 0;
   while (done < steps) {
-    const uint32_t k = std::min(E->steps_per_group, steps - done);
-    for (GroupArgs g : E->groups) {
+    const uint32_t k = std::min(per_group, steps - done);
+    for (GroupArgs g : groups) {
       // at most kMaxEnsembleBlocks persistent blocks per launch
       g.tiles_per_block = std::max(E->tiles_per_block,
                                    (g.ntiles + kMaxEnsembleBlocks - 1) / kMaxEnsembleBlocks);
@@ -3997,7 +4028,7 @@ olbgfx_status ensemble_enqueue(olbgfx_ensemble* E, uint32_t steps, hipStream_t s
       const dim3 grid(8 * g.blocks_per_xcd), block(E->block_threads);
       const uint32_t nm = (g.member_end - g.member_begin) * Q;
       for (uint32_t j = 0; j < k; ++j) {
-        ensemble_kernel<S><<<grid, block, E->lds, stream>>>((const StepArgs<A>*)E->args_dev,
+        ensemble_kernel<S><<<grid, block, lds, stream>>>((const StepArgs<A>*)E->args_dev,
                                                             E->tiles_dev, g, E->shift_ptrs_dev,
                                                             E->dmod_dev, E->counts_dev);
         if (!E->ticket) {
@@ -4112,6 +4143,7 @@ olbgfx_status olbgfx_ensemble_set_launch(olbgfx_ensemble* E, uint32_t block_thre
   E->block_threads = block_threads;
   E->waves_per_simd = waves_per_simd;
   E->tiles_per_block = tiles_per_block;
+  E->launch_given = true;
   E->lds = lds_for(block_threads, waves_per_simd);
   drop_graph(E);
   return OLBGFX_OK;
@@ -4139,6 +4171,7 @@ olbgfx_status olbgfx_ensemble_set_schedule(olbgfx_ensemble* E, uint64_t group_by
   if (steps_per_group == 0 || steps_per_group > 1024) {
     return fail(OLBGFX_ERR_INVALID, "steps per group must be in [1, 1024]");
   }
+  E->schedule_given = true;
   E->group_bytes = group_bytes;
   E->steps_per_group = steps_per_group;
   E->ticket = ticket ? 1 : 0;
@@ -5022,8 +5055,8 @@ olbgfx_status olbgfx_autotune_ensemble(olbgfx_ensemble* E, uint32_t steps, const
   static const uint32_t kBlocks[] = {128, 256};
   static const uint32_t kWaves[] = {0, 3, 4, 5};
   static const uint32_t kTiles[] = {1, 2, 4};
-  static const uint64_t kGroups[] = {0, 96ull << 20, 160ull << 20};
-  static const uint32_t kPerGroup[] = {1, 4, 8};
+  static const uint64_t kGroups[] = {0, 160ull << 20, kGroupBytes};
+  static const uint32_t kPerGroup[] = {1, 8, 64};
   static const int32_t kTickets[] = {0, 1};
   const olbgfx_tune_space none{};
   const olbgfx_tune_space& sp = space ? *space : none;
