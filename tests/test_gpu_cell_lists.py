@@ -3,6 +3,7 @@ scattered against the populations the lattice hands out: exact, in every
 storage type."""
 import numpy as np
 import pytest
+import torch  # before the library, so that both use one HIP runtime
 
 from openlb_amd import Lattice
 
@@ -14,8 +15,6 @@ WORD = {"f32": np.uint32, "f16": np.uint16, "bf16": np.uint16, "f64": np.uint64}
 @pytest.mark.parametrize("n", [1, 63, 255, 256, 257, 1000])
 @pytest.mark.parametrize("storage", ["f32", "f16", "bf16", "f64"])
 def test_gather_and_scatter(storage, n):
-    import torch
-
     print(f"[cells] {storage} n={n}", flush=True)
     rng = np.random.default_rng(n)
     a, b = (Lattice((9, 8, 11), 2, (True, False, True), storage) for _ in range(2))
