@@ -287,8 +287,8 @@ olbgfx_status olbgfx_reduce_moments(olbgfx_lattice* lattice, double out[8], void
  * and returns the same values bit for bit.  Lattices of more than 2^24 core
  * cells (65536 blocks of 256) are refused with OLBGFX_ERR_INVALID.  It calls
  * no hipMalloc or hipFree.  Calls within one process are serialised on a
- * lock, since every call on a device shares that device's array, which
- * keeps the last call's partial sums.  Synchronises. */
+ * lock, since every call on a device shares that device's array; the sums of
+ * its rows are taken on the device.  Synchronises. */
 olbgfx_status olbgfx_reduce_moments_noalloc(olbgfx_lattice* lattice, double out[8], void* stream);
 
 /* density and velocity of every padded cell through the momenta of its
