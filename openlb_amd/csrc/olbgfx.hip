@@ -1607,9 +1607,10 @@ __global__ void __launch_bounds__(256) residual_kernel(const StepArgs<typename S
 // tiles_per_block tiles of the group, with the XCD-aware order of the
 // single-lattice kernel.  Member descriptors and ring offsets live in device
 // memory, so the launch has fixed arguments and can be replayed from a
-// captured graph.  The last block to finish (ticket counter) advances the
-// ring offsets of the group's members, s_i -= d_i (mod ncells), for the next
-// launch; the counter is left at zero for it.
+// captured graph.  The offsets of up to kShiftRows steps are formed by one
+// launch before them (advance_shifts).  With the ticket, the last block to
+// finish advances the ring offsets of the group's members, s_i -= d_i (mod
+// ncells), for the next launch and leaves the counter at zero for it.
 
 struct Tile {
   uint32_t member;
@@ -1617,7 +1618,7 @@ struct Tile {
 };
 
 struct GroupArgs {
-  uint32_t ticket;           // 1: the last block advances the offsets (else a separate kernel)
+  uint32_t ticket;           // 1: the last block advances the offsets (else advance_shifts has, into rows)
   uint32_t tile_begin;       // first tile of the group
   uint32_t ntiles;           // tiles of the group
   uint32_t member_begin;     // members [member_begin, member_end) form the group
@@ -1627,6 +1628,7 @@ struct GroupArgs {
   uint32_t blocks_per_xcd;   // rounded up to whole runs
   int32_t xcd_run_log2;      // block order, as in the step kernel
   uint32_t* counter;         // ticket counter of the group (0 between launches)
+  const uint32_t* rows;      // this step's offsets of all members (null: their own arrays)
 };
 
 template <typename S>
@@ -1644,9 +1646,10 @@ __global__ void __launch_bounds__(kMaxBlock)
     for (uint32_t t = t0; t < t1; ++t) {
       const Tile tile = tiles[t];
       const StepArgs<A>& a = members[tile.member];
+      const uint32_t* from = g.rows ? g.rows + tile.member * Q : a.shift_dev;
       uint32_t sh[Q];
 #pragma unroll
-      for (int i = 0; i < Q; ++i) sh[i] = a.shift_dev[i];
+      for (int i = 0; i < Q; ++i) sh[i] = from[i];
       const uint32_t lin = tile.first + threadIdx.x;
       A st_rho, st_usqr;
       bool counted = false;
@@ -1678,15 +1681,28 @@ __global__ void __launch_bounds__(kMaxBlock)
   }
 }
 
-// advance the ring offsets of members [begin, end): s_i -= d_i (mod ncells)
+// Advances the ring offsets of members [begin, end) by `steps` steps, s_i -= d_i
+// (mod ncells) each, and leaves those of step j in row j of `rows`, where that
+// step's launch reads them.  A launch after every step for the next one's
+// offsets took 4.8 us of the 58 that a step of a 200 MiB group takes, all of it
+// latency.  64 cavities with edges in 32..128, us a step in calls
+// of 20: FP32 1216 -> 1170, FP16 711 -> 695
+constexpr uint32_t kShiftRows = 32;
+
 __global__ void advance_shifts(uint32_t* const* shifts, const uint32_t* dmod, const uint32_t* counts,
-                               uint32_t begin, uint32_t end)
+                               uint32_t begin, uint32_t end, uint32_t steps, uint32_t* rows, uint32_t row)
 {
   const uint32_t k = begin * Q + blockIdx.x * blockDim.x + threadIdx.x;
   if (k < end * Q) {
     const uint32_t l = k / Q, i = k % Q;
-    const uint64_t s = (uint64_t)shifts[l][i] + dmod[k];
-    shifts[l][i] = (uint32_t)(s >= counts[l] ? s - counts[l] : s);
+    const uint32_t d = dmod[k], count = counts[l];
+    uint32_t s = shifts[l][i];
+    for (uint32_t j = 0; j < steps; ++j) {
+      rows[(size_t)j * row + k] = s;
+      const uint64_t n = (uint64_t)s + d;
+      s = (uint32_t)(n >= count ? n - count : n);
+    }
+    shifts[l][i] = s;
   }
 }
 
@@ -3982,11 +3998,12 @@ olbgfx_status olbgfx_synchronize(olbgfx_lattice* L)
 // ensemble of independent lattices
 
 // Default schedule.  64 cavities of 32 to 128 cells a side, us an ensemble step
-// in calls of 20 steps: all members a launch FP32 1630, FP16 913; groups of 160,
-// 180, 208 and 240 MiB FP32 1259, 1238, 1231, 1257, FP16 744, 725, 716, 814
-// (smaller groups leave CUs idle, larger ones fall out of the cache).  A group
+// in calls of 20 steps: all members a launch FP32 1630, FP16 913; groups of 140,
+// 160, 180, 200 and 220 MiB FP32 1199, 1191, 1176, 1169, 1190, FP16 714, 710, 695,
+// 691, 689; of 240 MiB FP16 in calls with a launch a step for the offsets 814
+// against 716 of 208 (smaller groups leave CUs idle, larger ones fall out of the cache).  A group
 // has to come back to its rings a few times: groups of 208 MiB with 1, 2 and 4
-// steps each take FP32 1673, 1479, 1358, FP16 978, 947, 858.
+// steps each took FP32 1673, 1479, 1358, FP16 978, 947, 858 with such launches.
 constexpr uint64_t kGroupBytes = 200ull << 20;
 constexpr uint32_t kGroupSteps = 4;
 
@@ -4000,6 +4017,7 @@ struct olbgfx_ensemble {
   uint32_t** shift_ptrs_dev = nullptr;
   uint32_t* dmod_dev = nullptr;
   uint32_t* counts_dev = nullptr;
+  uint32_t* rows_dev = nullptr;      // kShiftRows steps' offsets of all members
   uint32_t block_threads = 256;
   uint32_t waves_per_simd = 0;
   uint32_t tiles_per_block = 1;
@@ -4016,7 +4034,7 @@ struct olbgfx_ensemble {
   uint64_t group_bytes = kGroupBytes;
   uint32_t steps_per_group = 1;
   bool schedule_given = false, launch_given = false;
-  uint32_t ticket = 0;               // 1: last block advances the offsets; 0: separate kernel
+  uint32_t ticket = 0;               // 1: last block advances the offsets; 0: advance_shifts, up to 32 steps at a time
   uint64_t grouped_bytes = ~0ull;
   std::vector<uint32_t> order;       // member index of each descriptor slot
   std::vector<GroupArgs> groups;
@@ -4122,6 +4140,9 @@ olbgfx_status ensemble_prepare(olbgfx_ensemble* E, bool force)
     HIP_TRY(device_alloc(&E->dmod_dev, sizeof(uint32_t) * m * Q));
     HIP_TRY(device_alloc(&E->counts_dev, sizeof(uint32_t) * m));
   }
+  if (!E->rows_dev) {
+    HIP_TRY(device_alloc(&E->rows_dev, sizeof(uint32_t) * m * Q * kShiftRows));
+  }
   if (tiles.size() > E->tiles_capacity) {
     if (E->tiles_dev) {
       HIP_TRY(hipFree(E->tiles_dev));
@@ -4172,7 +4193,6 @@ olbgfx_status ensemble_enqueue(olbgfx_ensemble* E, uint32_t steps, hipStream_t s
       all.ntiles = E->ntiles;
       all.member_end = groups.back().member_end;
       groups.assign(1, all);
-      per_group = 1;
       if (!E->launch_given) {
         // as in default_launch: all members FP32 1630 / 1552 us with 4 waves a
         // SIMD, FP16 913 / 891 with 5
@@ -4197,15 +4217,16 @@ olbgfx_status ensemble_enqueue(olbgfx_ensemble* E, uint32_t steps, hipStream_t s
       g.ticket = E->ticket;
       const dim3 grid(8 * g.blocks_per_xcd), block(E->block_threads);
       const uint32_t nm = (g.member_end - g.member_begin) * Q;
+      const uint32_t row = (uint32_t)E->members.size() * Q;
       for (uint32_t j = 0; j < k; ++j) {
-        ensemble_kernel<S><<<grid, block, lds, stream>>>((const StepArgs<A>*)E->args_dev,
-                                                            E->tiles_dev, g, E->shift_ptrs_dev,
-                                                            E->dmod_dev, E->counts_dev);
-        if (!E->ticket) {
-          advance_shifts<<<(nm + 255) / 256, 256, 0, stream>>>(E->shift_ptrs_dev, E->dmod_dev,
-                                                               E->counts_dev, g.member_begin,
-                                                               g.member_end);
+        if (!E->ticket && j % kShiftRows == 0) {
+          advance_shifts<<<(nm + 255) / 256, 256, 0, stream>>>(E->shift_ptrs_dev, E->dmod_dev, E->counts_dev,
+                                                               g.member_begin, g.member_end,
+                                                               std::min(kShiftRows, k - j), E->rows_dev, row);
         }
+        g.rows = E->ticket ? nullptr : E->rows_dev + (size_t)(j % kShiftRows) * row;
+        ensemble_kernel<S><<<grid, block, lds, stream>>>((const StepArgs<A>*)E->args_dev, E->tiles_dev, g,
+                                                         E->shift_ptrs_dev, E->dmod_dev, E->counts_dev);
       }
     }
     done += k;
@@ -4290,6 +4311,7 @@ olbgfx_status olbgfx_ensemble_destroy(olbgfx_ensemble* E)
   (void)hipFree(E->shift_ptrs_dev);
   (void)hipFree(E->dmod_dev);
   (void)hipFree(E->counts_dev);
+  (void)hipFree(E->rows_dev);
   (void)hipFree(E->counters_dev);
   delete E;
   return OLBGFX_OK;

@@ -30,8 +30,8 @@
 // a cache line.
 //
 // Measured on 512^3 BGK, us a step, against the single step: FP32 2765 / 4378,
-// FP16 1752 / 2220, BF16 1705 / 2249.  In FP32 a pass reads 1.53 times and
-// writes 1.05 times the populations at 4.7 TB/s; the copy of the same card
+// FP16 1752 / 2220, BF16 1705 / 2249.  In FP32 a pass reads 1.21 times and
+// writes 1.01 times the populations at 4.1 TB/s, the VALU 43 % busy; the copy of the same card
 // reaches 6.6, the single step in place 5.1.  The rest is the tiles' rims (1.33 x 1.13) and
 // their ragged cache lines.  Rows side by side gained 2.5 % in FP32 and 5 % in
 // FP16 over 19 separate rings; loading the next plane one turn of the sweep
