@@ -250,12 +250,12 @@ olbgfx_status olbgfx_set_populations(olbgfx_lattice* lattice, int32_t value_type
  * Four or more steps in one call take two steps a pass over the populations
  * where that is faster, on lattices that are periodic along every axis or
  * along none, without velocity-boundary or Bouzidi cells and without an
- * in-flight limit.  Results do not change (FP16 storage: up to the last bit),
- * except that the padding cells of a periodic lattice then hold no population
- * but those that enter or left the core.  Such a lattice keeps a second set of
- * populations from then on, if that takes at most a quarter of the free device
- * memory; an allocation of this library that would fail takes it back.  A
- * stream under capture takes single steps. */
+ * in-flight limit.  Results do not change, in any storage, however the steps
+ * are split into calls, except that the padding cells of a periodic lattice
+ * then hold no population but those that enter or left the core.  Such a
+ * lattice keeps a second set of populations from then on, if that takes at
+ * most a quarter of the free device memory; an allocation of this library that
+ * would fail takes it back.  A stream under capture takes single steps. */
 olbgfx_status olbgfx_collide_and_stream(olbgfx_lattice* lattice, uint32_t steps, void* stream);
 
 /* BlockLattice::postProcess() of the PostStream stage on the current

@@ -13,7 +13,7 @@
 // four workgroups; nothing is exchanged between them, so the populations go to
 // a second buffer.  Every value is rounded to the storage type between the
 // steps and every collision is that of the single step, so the two paths agree
-// bit for bit (FP16: to its last bit, where a conversion may fuse with an FMA).
+// bit for bit (in FP16 too: see pack_here).
 //
 // LDS holds 20 values a cell (80 KiB for 1024 threads in FP32): the four
 // populations that move against the sweep and across columns for one plane,
@@ -130,6 +130,20 @@ __device__ __forceinline__ ArgSegment<P> arguments_again()
   auto k = (ArgSegment<P>)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(k));
   return k;
+}
+
+// A population rounded to storage in the block that formed it.  The conversion
+// to FP16 fuses with the FMA that ends a collision, and rounds once, only where
+// both are in one block; the compiler moves a conversion whose result only the
+// second step reads into that step's branch, where it rounds twice.
+template <typename S>
+__device__ __forceinline__ S pack_here(typename Storage<S>::A v)
+{
+  S s = Storage<S>::pack(v);
+  if constexpr (std::is_same_v<S, f16_t>) {
+    asm volatile("" : "+v"(s.v));
+  }
+  return s;
 }
 
 // scalar base and 32-bit vector offset
@@ -270,10 +284,10 @@ __global__ void __launch_bounds__(NT) pair_kernel(const PairArgs<typename Storag
     }
     g[0] = rest;
     g[10] = ahead0;
-    g[1] = St::unpack(St::pack(f[1]));
-    rest = St::unpack(St::pack(f[0]));
+    g[1] = St::unpack(pack_here<S>(f[1]));
+    rest = St::unpack(pack_here<S>(f[0]));
     ahead0 = ahead1;
-    ahead1 = St::unpack(St::pack(f[10]));
+    ahead1 = St::unpack(pack_here<S>(f[10]));
     const int id2 = id_before;
     id_before = id;
     __syncthreads();

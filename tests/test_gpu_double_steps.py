@@ -1,0 +1,51 @@
+"""Runs that take two steps a pass in 2-byte storage against the same steps one
+a call, bit for bit: a conversion to FP16 that fuses with the last FMA of a
+collision in one kernel has to fuse in the other too.  Runs of 14 steps go
+through all three passes (rings to flat, flat to flat, flat to rings)."""
+import numpy as np
+import pytest
+import torch
+
+from openlb_amd import BGK, FORCED_TRT, Dynamics, Lattice
+
+pytestmark = pytest.mark.gpu
+
+KINDS = {"bgk": Dynamics(BGK, omega=1 / 0.6), "forced_trt": Dynamics(FORCED_TRT, omega=1.3, magic=0.2,
+                                                                     force=(1e-4, 0.0, -2e-5))}
+
+
+def _core(extent, padding):
+    mask = np.zeros(tuple(n + 2 * padding for n in extent), dtype=np.uint8)
+    mask[padding:-padding, padding:-padding, padding:-padding] = 1
+    return mask
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("extent", [(187, 190, 201), (1030, 257, 258)], ids=["7M", "68M"])
+def test_two_byte_runs(extent, storage, kind):
+    """both workgroup sizes: 1024 threads, and 512 from 64 M cells"""
+    print(f"[double steps] {storage} {kind} {extent}", flush=True)
+    mask = _core(extent, 1)
+    ids = np.flatnonzero(mask.reshape(-1)).astype(np.uint32)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16}[storage]
+    start = torch.empty((19, ids.size), dtype=dtype, device="cuda").normal_(0.0, 0.002, generator=gen)
+    torch.cuda.synchronize()
+    out = []
+    for calls in ([14, 5], [1] * 19):
+        lat = Lattice(extent, 1, (True,) * 3, storage)
+        lat.set_dynamics(1, KINDS[kind])
+        lat.set_dynamics_mask(mask)
+        cells = lat.cell_list(ids)
+        lat.scatter_cells(cells, start.data_ptr())
+        for steps in calls:
+            lat.collide_and_stream(steps)
+        got = torch.empty_like(start)
+        lat.gather_cells(cells, got.data_ptr())
+        lat.synchronize()
+        out.append(got.view(torch.int16))
+        cells.close()
+        lat.close()
+    assert torch.equal(out[0], out[1])
