@@ -2132,11 +2132,15 @@ uint32_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
 // / 1018; porous channel FP16 125 / 120.  Between 256 MiB and 1 GiB contiguous
 // parts stay better in 4-byte storage (40x300x400 capped: 138 against 144, 150
 // without the cap), and below 224 MiB the cache serves them best (160^3 FP16
-// 47 against 49, cavity 33^3 FP32 4.8 against 5.3).
+// 47 against 49, cavity 33^3 FP32 4.8 against 5.3).  Velocity and pressure
+// boundaries hide their chains of loads behind other waves, so steps with them
+// take no cap (LocalVelocity cavity FP32, capped / uncapped: 150^3 162 / 141,
+// 200^3 331 / 314, 240^3 560 / 526).
 void default_launch(const olbgfx_lattice* L, uint32_t& lds, int32_t& order)
 {
   const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
-  lds = L->launch_given ? L->lds_reserve : (L->elem == 4 && mib >= 256 ? lds_for(L->block_threads, 4) : 0);
+  const bool capped = L->elem == 4 && mib >= 256 && !L->boundary_kinds;
+  lds = L->launch_given ? L->lds_reserve : (capped ? lds_for(L->block_threads, 4) : 0);
   if (L->order_given) {
     order = L->xcd_run_log2;
   } else if (L->elem == 2) {
