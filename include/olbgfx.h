@@ -252,11 +252,23 @@ olbgfx_status olbgfx_set_populations(olbgfx_lattice* lattice, int32_t value_type
  * along none, without velocity-boundary or Bouzidi cells and without an
  * in-flight limit.  Results do not change, in any storage, however the steps
  * are split into calls, except that the padding cells of a periodic lattice
- * then hold no population but those that enter or left the core.  Such a
- * lattice keeps a second set of populations from then on, if that takes at
- * most a quarter of the free device memory; an allocation of this library that
- * would fail takes it back.  A stream under capture takes single steps. */
+ * then hold no population but those that enter or left the core.  The first
+ * such run allocates a second set of populations, which the lattice keeps
+ * (olbgfx_set_two_step).  A stream under capture takes single steps. */
 olbgfx_status olbgfx_collide_and_stream(olbgfx_lattice* lattice, uint32_t steps, void* stream);
+
+/* Device memory that a lattice may hold for runs of two steps a pass: a lattice
+ * whose second set of populations is larger than max_bytes, or than a quarter
+ * of the free device memory when it is allocated, takes single steps.
+ * UINT64_MAX until this is called; with 0 the lattice takes single steps from
+ * now on.  A set that is held and larger is given back before the call returns,
+ * which waits for the device; an allocation of this library that would fail
+ * gives the sets of all lattices back too.  No reference counterpart. */
+olbgfx_status olbgfx_set_two_step(olbgfx_lattice* lattice, uint64_t max_bytes);
+
+/* the bytes of the second set held now (0: none), and how many steps were so
+ * far taken two a pass */
+olbgfx_status olbgfx_get_two_step(olbgfx_lattice* lattice, uint64_t* bytes, uint64_t* steps);
 
 /* BlockLattice::postProcess() of the PostStream stage on the current
  * populations, without a step: the Bouzidi, LocalVelocity edge and corner

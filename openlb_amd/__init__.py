@@ -100,6 +100,8 @@ def library() -> ctypes.CDLL:
         "olbgfx_device_count": [ctypes.POINTER(i32)],
         "olbgfx_set_split": [vp, i32],
         "olbgfx_get_split": [vp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_uint32)],
+        "olbgfx_set_two_step": [vp, ctypes.c_uint64],
+        "olbgfx_get_two_step": [vp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)],
         "olbgfx_probe_bandwidth": [ctypes.POINTER(_LatticeDesc), i32, u32, i32, u32, vp,
                                    ctypes.POINTER(ctypes.c_double)],
         "olbgfx_set_inflight_limit": [vp, u32],
@@ -378,6 +380,19 @@ class Lattice:
         kind, rest = ctypes.c_int32(), ctypes.c_uint32()
         _check(library().olbgfx_get_split(self._h, ctypes.byref(kind), ctypes.byref(rest)))
         return kind.value, rest.value
+
+    def set_two_step(self, max_bytes: int | None = None) -> None:
+        """device memory this lattice may hold for runs of steps that are
+        taken two a pass, never more than a quarter of what is free; None: no
+        other limit, 0: single steps only.  What is held and larger is given
+        back."""
+        _check(library().olbgfx_set_two_step(self._h, (1 << 64) - 1 if max_bytes is None else int(max_bytes)))
+
+    def get_two_step(self) -> tuple:
+        """(bytes held for such runs, steps taken two a pass so far)"""
+        held, steps = ctypes.c_uint64(), ctypes.c_uint64()
+        _check(library().olbgfx_get_two_step(self._h, ctypes.byref(held), ctypes.byref(steps)))
+        return held.value, steps.value
 
     def set_block_order(self, xcd_run_log2: int = -1) -> None:
         """-1: each XCD sweeps one contiguous part; k: XCDs take turns on runs

@@ -2028,10 +2028,13 @@ struct olbgfx_lattice {
   uint64_t split_version = ~0ull;
   bool split_enabled = true;         // olbgfx_set_split
   // second set of populations, which passes of two steps write to: held from
-  // the first run of steps that takes them until the lattice is destroyed or
-  // an allocation needs the memory
+  // the first run of steps that takes them until the lattice is destroyed, an
+  // allocation needs the memory or olbgfx_set_two_step takes it back
   void* pair_pop = nullptr;
   int pair_device = 0;
+  uint64_t pair_limit = ~0ull;       // olbgfx_set_two_step
+  uint32_t pair_refused = 0;         // runs left before the memory is asked for again
+  uint64_t pair_steps = 0;           // steps so far that were taken two a pass
   PairPlan pair_plan;
   bool walls_only = false;           // wall_mode, as of wall_version
   uint64_t wall_version = ~0ull;
@@ -2433,8 +2436,11 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
 }
 
 // the lattice's second set of populations; false where it cannot be had: the
-// stream is being captured, or it would take more than a quarter of the free
-// device memory
+// stream is being captured, it is larger than the lattice may hold, or it would
+// take more than a quarter of the free device memory, which is asked for again
+// kPairRetry runs later
+constexpr uint32_t kPairRetry = 64;
+
 bool prepare_pair(olbgfx_lattice* L, hipStream_t stream)
 {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -2444,11 +2450,19 @@ bool prepare_pair(olbgfx_lattice* L, hipStream_t stream)
   }
   if (!L->pair_pop) {
     const size_t bytes = (size_t)Q * L->stride * L->elem;
+    if (bytes > L->pair_limit) {
+      return false;
+    }
+    if (L->pair_refused > 0) {
+      --L->pair_refused;
+      return false;
+    }
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > free_bytes / 4 ||
         hipMalloc(&L->pair_pop, bytes) != hipSuccess) {
       (void)hipGetLastError();
       L->pair_pop = nullptr;
+      L->pair_refused = kPairRetry - 1;
       return false;
     }
     (void)hipGetDevice(&L->pair_device);
@@ -2641,6 +2655,7 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
     if (L->stats_partial) {
       HIP_TRY(hipFree(L->stats_partial));
       L->stats_partial = nullptr;
+      L->stats_capacity = 0;
     }
     const uint32_t sums = (a.nblocks + kStatsChunk - 1) / kStatsChunk;
     HIP_TRY(device_alloc(&L->stats_partial, 4 * sizeof(double) * ((size_t)a.nblocks + sums)));
@@ -2706,6 +2721,7 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
       std::swap(rings[0], rings[1]);
     }
     a.pop = L->pop;
+    L->pair_steps += first;
   }
   for (uint32_t k = first; k < steps; ++k) {
     for (int i = 0; i < Q; ++i) a.shift[i] = L->shift[i];
@@ -3971,6 +3987,32 @@ olbgfx_status olbgfx_set_launch(olbgfx_lattice* L, uint32_t block_threads, uint3
   L->block_threads = block_threads;
   L->lds_reserve = lds_for(block_threads, waves_per_simd);
   L->launch_given = true;
+  return OLBGFX_OK;
+}
+
+olbgfx_status olbgfx_set_two_step(olbgfx_lattice* L, uint64_t max_bytes)
+{
+  if (check(L) != OLBGFX_OK) {
+    return OLBGFX_ERR_INVALID;
+  }
+  // no run of another thread is being enqueued while it is given back
+  std::unique_lock<std::shared_mutex> alone(g_pair_use);
+  L->pair_limit = max_bytes;
+  L->pair_refused = 0;
+  if (L->pair_pop && (uint64_t)Q * L->stride * L->elem > max_bytes) {
+    drop_pair_buffer(L);  // waits for the device
+  }
+  return OLBGFX_OK;
+}
+
+olbgfx_status olbgfx_get_two_step(olbgfx_lattice* L, uint64_t* bytes, uint64_t* steps)
+{
+  if (check(L) != OLBGFX_OK || !bytes || !steps) {
+    return fail(OLBGFX_ERR_INVALID, "null argument");
+  }
+  std::lock_guard<std::mutex> lock(g_pair_list);
+  *bytes = L->pair_pop ? (uint64_t)Q * L->stride * L->elem : 0;
+  *steps = L->pair_steps;
   return OLBGFX_OK;
 }
 

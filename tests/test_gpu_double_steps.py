@@ -1,12 +1,13 @@
-"""Runs that take two steps a pass in 2-byte storage against the same steps one
-a call, bit for bit: a conversion to FP16 that fuses with the last FMA of a
-collision in one kernel has to fuse in the other too.  Runs of 14 steps go
-through all three passes (rings to flat, flat to flat, flat to rings)."""
+"""Runs that take two steps a pass: in 2-byte storage against the same steps one
+a call, bit for bit (a conversion to FP16 that fuses with the last FMA of a
+collision in one kernel has to fuse in the other too), and what they do with
+memory.  Runs of 14 steps go through all three passes (rings to flat, flat to
+flat, flat to rings)."""
 import numpy as np
 import pytest
 import torch
 
-from openlb_amd import BGK, FORCED_TRT, Dynamics, Lattice
+from openlb_amd import BGK, FORCED_TRT, Dynamics, Lattice, cases
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,40 @@ def test_two_byte_runs(extent, storage, kind):
         cells.close()
         lat.close()
     assert torch.equal(out[0], out[1])
+
+
+def _tgv(n):
+    case = cases.tgv(n, dtype=np.float32)
+    lat = Lattice(case.extent, case.padding, case.periodic, "f32")
+    case.apply(lat)
+    return case, lat
+
+
+def test_second_set_is_limited_and_given_back():
+    print("[double steps] memory", flush=True)
+    case, lat = _tgv(160)
+    _, single = _tgv(160)
+    single.set_two_step(0)
+    size = 19 * 4 * lat.ncells
+    free = torch.cuda.mem_get_info()[0]
+    lat.collide_and_stream(8)
+    held, steps = lat.get_two_step()
+    assert held >= size and steps == 8
+    lat.synchronize()
+    assert torch.cuda.mem_get_info()[0] <= free - size
+    lat.set_two_step(held)                      # fits: kept
+    assert lat.get_two_step() == (held, 8)
+    lat.set_two_step(held - 1)                  # given back, and not taken again
+    assert lat.get_two_step() == (0, 8)
+    assert torch.cuda.mem_get_info()[0] >= free - size // 8
+    lat.collide_and_stream(6)
+    assert lat.get_two_step() == (0, 8)
+    lat.set_two_step()
+    lat.collide_and_stream(7)
+    assert lat.get_two_step() == (held, 12)
+    single.collide_and_stream(21)
+    assert single.get_two_step() == (0, 0)
+    core = case.core_mask().reshape(-1)
+    np.testing.assert_array_equal(lat.get_populations()[:, core], single.get_populations()[:, core])
+    lat.close()
+    single.close()
