@@ -2435,6 +2435,26 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
   return beyond_cache || (bgk && cells >= 2400000) ? 1024 : 0;
 }
 
+// While it lives, calls that may not be recorded (an allocation) leave the
+// captures of other threads alone, where they would otherwise end them with an
+// error; this thread must not be capturing.
+class OutsideCaptures {
+ public:
+  OutsideCaptures() { held_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+  ~OutsideCaptures()
+  {
+    if (held_) {
+      (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+  }
+  OutsideCaptures(const OutsideCaptures&) = delete;
+  OutsideCaptures& operator=(const OutsideCaptures&) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  bool held_ = false;
+};
+
 // the lattice's second set of populations; false where it cannot be had: the
 // stream is being captured, it is larger than the lattice may hold, or it would
 // take more than a quarter of the free device memory, which is asked for again
@@ -2457,6 +2477,7 @@ bool prepare_pair(olbgfx_lattice* L, hipStream_t stream)
       --L->pair_refused;
       return false;
     }
+    const OutsideCaptures outside;
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > free_bytes / 4 ||
         hipMalloc(&L->pair_pop, bytes) != hipSuccess) {

@@ -3,6 +3,8 @@ a call, bit for bit (a conversion to FP16 that fuses with the last FMA of a
 collision in one kernel has to fuse in the other too), and what they do with
 memory.  Runs of 14 steps go through all three passes (rings to flat, flat to
 flat, flat to rings)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -87,3 +89,43 @@ def test_second_set_is_limited_and_given_back():
     np.testing.assert_array_equal(lat.get_populations()[:, core], single.get_populations()[:, core])
     lat.close()
     single.close()
+
+
+def test_first_run_leaves_a_capture_of_another_thread_alone():
+    """the first run of a lattice allocates; a stream that another thread is
+    capturing must not notice"""
+    print("[double steps] another thread captures", flush=True)
+    case, lat = _tgv(64)
+    _, ref = _tgv(64)
+    ref.collide_and_stream(8)
+    ref.synchronize()
+    side, own = torch.cuda.Stream(), torch.cuda.Stream()
+    x = torch.zeros(256, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    errors = []
+
+    def run():
+        try:
+            lat.collide_and_stream(8, own.cuda_stream)
+        except Exception as exc:
+            errors.append(exc)
+
+    with torch.cuda.graph(graph, stream=side, capture_error_mode="global"):
+        x.add_(1.0)
+        thread = threading.Thread(target=run)
+        thread.start()
+        thread.join()
+        x.add_(1.0)
+    assert not errors
+    own.synchronize()
+    x.zero_()
+    for k in (1, 2, 3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert x.tolist() == [2.0 * k] * 256
+    assert lat.get_two_step()[1] == 8
+    core = case.core_mask().reshape(-1)
+    np.testing.assert_array_equal(lat.get_populations()[:, core], ref.get_populations()[:, core])
+    lat.close()
+    ref.close()
