@@ -248,7 +248,7 @@ olbgfx_status olbgfx_set_populations(olbgfx_lattice* lattice, int32_t value_type
  * Enqueued on `stream`; does not synchronise.
  *
  * Four or more steps in one call take two steps a pass over the populations
- * where that is faster, on lattices that are periodic along every axis or
+ * where that is faster (by size, kind and number of steps), on lattices that are periodic along every axis or
  * along none, without velocity-boundary or Bouzidi cells and without an
  * in-flight limit.  Results do not change, in any storage, however the steps
  * are split into calls, except that the padding cells of a periodic lattice

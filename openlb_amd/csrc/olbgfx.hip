@@ -1955,6 +1955,7 @@ struct PairPlan {
   uint32_t threads = 0;  // 0: not chosen yet
   uint32_t tz = 0, ty = 0, ntz = 0, nty = 0, xlen = 0, nwork = 0;
   bool worth = false;
+  double turns = 0;  // turns of a lane on the busiest CU for each cell of its share (pair_pays)
 };
 
 struct olbgfx_lattice {
@@ -2393,20 +2394,21 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
 // runs of steps, two steps a pass (olbgfx_pair.h)
 
 // Workgroup size of the two-step kernel for this lattice, or 0 where single
-// steps are faster; mode is the kind of a uniform lattice or -1.  Two steps a
-// pass halve the traffic to HBM but do the first step of every tile's rim
-// twice, so they win where HBM bounds the single step: from 256 MiB of
-// populations, the size of the Infinity Cache (us a step, single / two a pass:
-// BGK 160^3 FP32 132 / 86, 512^3 FP32 4378 / 2765, FP16 2220 / 1752, BF16
-// 2249 / 1705; the porous channel 384x128x128 FP32 221 / 149; a closed cavity
-// 256^3 FP32 551 / 404, 200^3 FP64 515 / 375).  Below that size they win only
-// for uniform BGK, where the pass is short enough that the saved launch and
-// the saved round trip to the cache count: FP32 64^3 8.5 / 7.2, 101^3 27.5 /
-// 16.6, 140^3 64.5 / 56.4, but 128^3 47.2 / 48.3 in runs of 8 steps; FP64 64^3
-// 14.3 / 11.9.  Masked cells and
-// Smagorinsky BGK in 2-byte storage are bound by instruction issue: the former
-// lose (porous channel FP16 124 / 133), the latter gain 7 % in long runs and
-// lose 8 % in runs of 8 steps, whose first and last pass convert the layout.
+// steps are faster in runs of any length; mode is the kind of a uniform lattice
+// or that of wall_mode.  Two steps a pass halve the traffic to HBM but do the
+// first step of every tile's rim twice, so they win where HBM bounds the single
+// step: where the populations outgrow the Infinity Cache (us a step, single /
+// two a pass: BGK 160^3 FP32 132 / 86, 512^3 FP32 4378 / 2765, FP16 2220 /
+// 1752, BF16 2249 / 1705; the porous channel 384x128x128 FP32 221 / 149; a
+// closed cavity 256^3 FP32 551 / 404, 200^3 FP64 515 / 375).  Below that size
+// they win only for uniform BGK, and there while both sets of populations lie
+// in the cache: FP32 64^3 8.5 / 7.2, 101^3 27.5 / 16.6; FP64 64^3 14.3 / 11.9,
+// 100^3 43.5 / 41.  Between the two the second set drives the first out: FP32
+// boxes of 2.4 to 3.0 M cells take 0.86 to 1.24 of the single step's time, FP64
+// boxes of 180 to 255 MiB 0.9 to 1.17.  Masked cells and Smagorinsky BGK in
+// 2-byte storage are bound by instruction issue: the former lose (porous
+// channel FP16 124 / 133), the latter gain 7 % in long runs and lose 8 % in runs
+// of 8 steps, whose first and last pass convert the layout.
 // 1024 threads keep the rim small; 512 give more workgroups to small lattices
 // (101^3 FP32 16.6 against 18.0) and, in 2-byte storage, a second workgroup on
 // each CU, which pays for the larger rim in the largest lattices (512^3 FP16
@@ -2417,22 +2419,80 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
   const bool masked = mode < 0 || mode >= kWithWalls;
   const olbgfx_lattice_desc& D = L->desc;
   const uint64_t cells = (uint64_t)D.nx * D.ny * D.nz;
-  const uint64_t bytes = (uint64_t)Q * L->stride * L->elem;
-  const bool beyond_cache = bytes >= (256ull << 20);
+  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
   const bool bgk = mode == OLBGFX_BGK;
   if (L->elem == 2) {
-    if (masked || mode == OLBGFX_SMAGORINSKY_BGK || !beyond_cache) {
+    // BF16 ForcedTRT still gains from the cache at 257 MiB (165x245x159 1.18)
+    const bool late = mode == OLBGFX_FORCED_TRT && L->desc.storage == OLBGFX_STORE_BF16;
+    if (masked || mode == OLBGFX_SMAGORINSKY_BGK || mib < (late ? 272 : 256)) {
       return 0;
     }
     return cells >= (64u << 20) || (bgk && L->desc.storage == OLBGFX_STORE_BF16) ? 512 : 1024;
   }
   if (L->elem == 8) {
-    return beyond_cache || (bgk && bytes >= (48ull << 20)) ? 512 : 0;
+    return mib >= 260 || (bgk && mib >= 48 && mib < 176) ? 512 : 0;
   }
-  if (bgk && cells >= 60000 && cells < 1500000) {
-    return 512;
+  if (bgk && cells < 1500000) {
+    return cells >= 60000 ? 512 : 0;
   }
-  return beyond_cache || (bgk && cells >= 2400000) ? 1024 : 0;
+  return mib >= 256 ? 1024 : 0;
+}
+
+// Do runs that take `steps` steps (a multiple of four) in pairs win with these
+// tiles?  The first and the last pass convert the layout and cost more than the
+// others, and up to three single steps follow them on a cache that the second
+// set has filled, so where the gain is small short runs lose.  plan.turns is
+// what decides otherwise: the turns of a lane for each cell, that is 1 + the
+// share of rims, of lanes outside the lattice and of CUs left idle by the last
+// round.  Measured on 1300 random boxes, thin ones among them, in runs of 4 to
+// 100 steps against single steps; every rule below ends where a run of some
+// length took more than 1.02 of the single steps' time:
+// - FP32 BGK below 220000 cells: 48^3 6.1 us a step, 6.2 to 6.4 in pairs, 56^3
+//   7.2 / 8.1, but 44^3 6.0 / 5.1 and 52^3 6.8 / 6.4, whose tiles sweep a single
+//   plane with one workgroup a CU, or with enough cells for two.  Up to 400000
+//   cells in tiles of three planes and more, runs of 5 steps up to 1.04.
+// - FP64 from 128 to 176 MiB runs of 5 steps 1.04, of 9 1.03, of 12 and more 0.73
+//   to 0.98; up to 340 MiB other kinds than BGK 1.05 in runs of 5 steps, BGK on
+//   lattices thin along x or y 1.16.
+// - FP64 ForcedTRT above 3.0 turns 1.02 to 1.11, general masks above 2.8 turns
+//   1.02 to 1.13.
+// - Closed lattices thin along x or y, whose padding planes are updated too:
+//   FP32 4x1766x1766 1.05, 2218x8x2218 1.09; FP64 5x674x674 1.21.
+// - FP16 BGK with 1024 threads: runs of 4 steps 0.85 to 1.11, of 8 to 12 0.81 to
+//   0.99 up to 2 turns, 1.04 above; short rows in runs of any length 1057x1057x8
+//   1.16, 711x711x16 1.12, with ForcedTRT 1963x1963x4 1.12.
+// - BF16 ForcedTRT with 1024 threads: runs of 8 steps 0.88 to 1.06, of 12 and
+//   more 0.81 to 1.00 up to 1.75 turns, 1.03 above.
+bool pair_pays(const olbgfx_lattice* L, int mode, const PairPlan& plan, uint32_t steps)
+{
+  const olbgfx_lattice_desc& D = L->desc;
+  const uint64_t cells = (uint64_t)D.nx * D.ny * D.nz;
+  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
+  const bool bgk = mode == OLBGFX_BGK, forced = mode == OLBGFX_FORCED_TRT;
+  const bool thin = D.nx < 16 || D.ny < 16;
+  if (!plan.worth || (thin && !D.periodic[0])) {
+    return false;
+  }
+  if (L->elem == 2) {
+    if (forced && D.nz < 16) {
+      return false;
+    }
+    if (plan.threads == 512 || (forced && D.storage == OLBGFX_STORE_F16)) {
+      return true;
+    }
+    return D.nz >= 32 && (forced ? steps >= 12 && plan.turns <= 1.75 && !thin : steps >= 8 && plan.turns <= 2.0);
+  }
+  if (L->elem == 8) {
+    if (mib < 260) {
+      return mib < 128 || steps >= 12;
+    }
+    return (mib >= 340 || (!thin && (bgk || steps >= 12))) && plan.turns <= (mode < 0 ? 2.8 : forced ? 3.0 : 1e9);
+  }
+  if (plan.threads == 512) {
+    return cells >= 220000 ? cells >= 400000 || plan.xlen < 3 || steps >= 8
+                           : plan.xlen == 1 && (plan.nwork <= 256 || cells >= 135000);
+  }
+  return plan.turns <= 3.0;
 }
 
 // While it lives, calls that may not be recorded (an allocation) leave the
@@ -2534,6 +2594,8 @@ void pair_tiles(PairPlan& plan, const olbgfx_lattice* L, uint32_t threads)
     }
   }
   plan.worth = dx >= 4 && (double)dy * dz >= 0.4 * ((double)plan.ntz * plan.nty * threads);
+  plan.turns = (double)((plan.nwork + slots - 1) / slots) * slots * (std::min(plan.xlen, dx) + 3) * threads /
+               ((double)D.nx * D.ny * D.nz);
   plan.threads = threads;
 }
 
@@ -2708,18 +2770,20 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
   // to the second buffer and to L->pop in turn.  The statistics are those of
   // the last step, which runs alone.
   const bool all = a.periodic == 7, none = a.periodic == 0;  // mixed axes take single steps
-  const bool pair_kind = all && (mode == OLBGFX_BGK || mode == OLBGFX_FORCED_TRT || mode == OLBGFX_SMAGORINSKY_BGK);
-  const int pair_mode = pair_kind ? mode : wall_mode(L);
-  uint32_t threads = 0;
-  if (L->pair_enabled && (all || none) && steps > 0 && !L->boundary_kinds && L->bz_n == 0 && L->bzv_n == 0 &&
-      L->inflight_limit == 0 && mode != OLBGFX_NO_DYNAMICS) {
-    threads = pair_threads(L, pair_mode);
+  const uint32_t in_pairs = steps == 0 ? 0 : (L->stats_on ? steps - 1 : steps) / 4 * 4;
+  int pair_mode = 0;
+  bool pairs = in_pairs > 0 && L->pair_enabled && (all || none) && !L->boundary_kinds && L->bz_n == 0 &&
+               L->bzv_n == 0 && L->inflight_limit == 0 && mode != OLBGFX_NO_DYNAMICS;
+  if (pairs) {
+    const bool kind = all && (mode == OLBGFX_BGK || mode == OLBGFX_FORCED_TRT || mode == OLBGFX_SMAGORINSKY_BGK);
+    pair_mode = kind ? mode : wall_mode(L);
+    const uint32_t threads = pair_threads(L, pair_mode);
     if (threads > 0 && L->pair_plan.threads != threads) {
       pair_tiles(L->pair_plan, L, threads);
     }
+    pairs = threads > 0 && pair_pays(L, pair_mode, L->pair_plan, in_pairs);
   }
-  const uint32_t in_pairs = (L->stats_on ? steps - 1 : steps) / 4 * 4;
-  if (threads > 0 && in_pairs > 0 && L->pair_plan.worth) {
+  if (pairs) {
     std::shared_lock<std::shared_mutex> use(g_pair_use);
     const uint32_t end = prepare_pair(L, stream) ? in_pairs : 0;
     auto advance = [&](uint32_t (&s)[Q]) {

@@ -7,7 +7,7 @@ import time
 import numpy as np
 import pytest
 
-from openlb_amd import Lattice, cases
+from openlb_amd import BGK, BOUNCE_BACK, FORCED_TRT, Dynamics, Lattice, cases
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +46,69 @@ def test_velocity_boundaries_take_no_occupancy_cap(res):
     for lat in lats:
         lat.close()
     assert default <= (1.07 if res == 150 else 1.05) * uncapped
+
+
+BULK = {"bgk": Dynamics(BGK, omega=1 / 0.6), "forced_trt": Dynamics(FORCED_TRT, omega=1.3, magic=0.2,
+                                                                   force=(1e-5, 0.0, 0.0))}
+
+
+def _box(storage, kind, extent, padding):
+    """a uniform periodic box, or one of BGK closed by bounce-back cells"""
+    lat = Lattice(extent, padding, (kind != "closed",) * 3, storage)
+    mask = np.zeros(tuple(n + 2 * padding for n in extent), dtype=np.uint8)
+    mask[tuple(slice(padding, -padding) for _ in range(3))] = 1
+    lat.set_dynamics(1, BULK.get(kind, BULK["bgk"]))
+    if kind == "closed":
+        lat.set_dynamics(2, Dynamics(BOUNCE_BACK))
+        mask[mask == 1] = 2
+        mask[tuple(slice(padding + 1, -padding - 1) for _ in range(3))] = 1
+    lat.set_dynamics_mask(mask)
+    return lat
+
+
+# runs that took 1.08 to 1.2 of the single steps' time two steps a pass
+LOSERS = [("f32", "bgk", (56, 56, 56), 1, 8), ("f32", "bgk", (145, 109, 171), 3, 20),
+          ("f32", "bgk", (206, 82, 165), 1, 5), ("f32", "bgk", (132, 155, 151), 3, 20), ("f64", "bgk", (123, 90, 129), 3, 8),
+          ("f64", "bgk", (547, 4, 547), 1, 5), ("f64", "closed", (5, 674, 674), 1, 20),
+          ("f16", "bgk", (1057, 1057, 8), 1, 20), ("f16", "bgk", (89, 522, 212), 1, 4), ("f16", "forced_trt", (1963, 1963, 4), 1, 8),
+          ("bf16", "forced_trt", (207, 227, 312), 1, 4), ("bf16", "forced_trt", (165, 245, 159), 3, 20)]
+
+
+@pytest.mark.parametrize("storage,kind,extent,padding,steps", LOSERS)
+def test_runs_are_not_slower_than_single_steps(storage, kind, extent, padding, steps):
+    print(f"[launch defaults] {storage} {kind} {extent} runs of {steps}", flush=True)
+    lats = [_box(storage, kind, extent, padding) for _ in range(2)]
+    lats[1].set_two_step(0)
+    cells = int(np.prod(extent))
+    calls = max(2, int(2e8 / (cells * steps)))
+
+    def run(lat):
+        for _ in range(calls):
+            lat.collide_and_stream(steps)
+        lat.synchronize()
+
+    for lat in lats:
+        run(lat)
+    default, single = least([lambda: run(lats[0]), lambda: run(lats[1])])
+    for lat in lats:
+        lat.close()
+    assert default <= 1.045 * single
+
+
+@pytest.mark.parametrize("storage,kind,extent,padding,steps,pairs", [
+    ("f32", "bgk", (44, 44, 44), 1, 4, 4), ("f32", "bgk", (64, 64, 64), 3, 7, 4), ("f32", "bgk", (101, 101, 101), 1, 8, 8),
+    ("f32", "bgk", (160, 160, 160), 3, 5, 4), ("f32", "closed", (160, 160, 160), 1, 4, 4),
+    ("f64", "bgk", (72, 72, 72), 1, 4, 4), ("f64", "bgk", (94, 94, 94), 1, 13, 12), ("f64", "bgk", (140, 140, 140), 1, 4, 4),
+    ("f16", "bgk", (220, 220, 220), 1, 9, 8), ("f16", "forced_trt", (193, 193, 193), 1, 4, 4),
+    ("bf16", "bgk", (193, 193, 193), 1, 4, 4), ("bf16", "forced_trt", (344, 250, 86), 1, 12, 12),
+    ("f64", "bgk", (94, 94, 94), 1, 11, 0), ("f16", "bgk", (220, 220, 220), 1, 7, 0),
+    ("bf16", "forced_trt", (344, 250, 86), 1, 11, 0)])
+def test_steps_taken_two_a_pass(storage, kind, extent, padding, steps, pairs):
+    """both sides of the rules"""
+    print(f"[launch defaults] {storage} {kind} {extent} {steps} steps", flush=True)
+    lat = _box(storage, kind, extent, padding)
+    lat.collide_and_stream(steps)
+    lat.synchronize()
+    taken = lat.get_two_step()[1]
+    lat.close()
+    assert taken == pairs
