@@ -2881,7 +2881,7 @@ class Download {
   hipError_t copy(void* host, const void* device, size_t bytes)
   {
     std::unique_lock<std::mutex> lock(busy_, std::try_to_lock);
-    if (bytes < kLeast || !lock.owns_lock() || known(host) || !ready()) {
+    if (bytes < kLeast || !lock.owns_lock() || known(host) || !ready(bytes)) {
       return hipMemcpy(host, device, bytes, hipMemcpyDeviceToHost);
     }
     const size_t chunks = (bytes + kSlot - 1) / kSlot;
@@ -2962,10 +2962,11 @@ class Download {
       (void)hipHostFree(pinned_);
       pinned_ = nullptr;
     }
+    without_ = 0;
   }
 
  private:
-  static constexpr size_t kSlot = 2 << 20, kSlots = 16, kLeast = 8 << 20, kThreads = 4;
+  static constexpr size_t kSlot = 2 << 20, kSlots = 16, kLeast = 8 << 20, kThreads = 4, kWorth = 128 << 20;
   static bool known(const void* p)
   {
     hipPointerAttribute_t a{};
@@ -2975,7 +2976,7 @@ class Download {
     (void)hipGetLastError();
     return false;
   }
-  bool ready()
+  bool ready(size_t bytes)
   {
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) {
@@ -2983,6 +2984,12 @@ class Download {
     }
     if (pinned_) {
       return device == device_;
+    }
+    // the ring takes 4 ms to allocate, which it saves on 64 to 150 MB: a program
+    // that makes one lattice after another and reads each once does without
+    without_ += bytes;
+    if (without_ < kWorth) {
+      return false;
     }
     device_ = device;
     if (hipHostMalloc((void**)&pinned_, kSlot * kSlots, hipHostMallocPortable) != hipSuccess) {
@@ -3006,6 +3013,7 @@ class Download {
     return true;
   }
   std::mutex busy_;
+  size_t without_ = 0;  // bytes copied without the ring since it was given back
   char* pinned_ = nullptr;
   hipEvent_t copied_[kSlots] = {};
   int device_ = 0;
