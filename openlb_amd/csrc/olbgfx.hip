@@ -4900,6 +4900,8 @@ olbgfx_status olbgfx_halo_unpack(olbgfx_lattice* L, int32_t axis, int32_t side, 
 struct olbgfx_cell_list {
   uint32_t* cells = nullptr;  // device copy of the CellIDs
   uint32_t n = 0;
+  uint32_t runs = 0;          // stretches of consecutive ids
+  uint32_t segments = 0;      // stretches of ids in one aligned block of 64
   uint32_t count = 0;         // padded cells of the lattice the list was made for
 };
 
@@ -4912,12 +4914,13 @@ struct CellCopyArgs {
 };
 
 // One thread a cell: its id is read once and its 19 loads are in flight
-// together, where one thread a value read every id 19 times and divided 64-bit
-// indices.  Bound by HBM.  All core cells of 512^3, before and after: gather
-// FP32 10667 / 3955 us (5.2 TB/s), FP16 9481 / 2111 us; scatter FP32 9425 /
-// 5452 us; 128^3 FP32 gather 156 / 43 us.  The buffer is not read again here,
-// so the gather stores past the caches (4018 us without); the scatter's loads
-// do so only in 8-byte storage (128^3 156 / 142 us; 512^3 FP32 5452 / 6104).
+// together, where one thread a value (k_cell_values) reads every id 19 times.
+// For long lists of neighbouring cells (per_cell), bound by HBM.  All core cells
+// of 512^3, against one thread a value: gather FP32 10667 / 3955 us (5.2 TB/s),
+// FP16 9481 / 2111 us; scatter FP32 9425 / 5452 us.  The buffer is not read
+// again here, so the gather stores past the caches (4018 us without); the
+// scatter's loads do so only in 8-byte storage (128^3 156 / 142 us; 512^3 FP32
+// 5452 / 6104).
 template <typename S, bool GATHER>
 __global__ void __launch_bounds__(256) k_cells(void* pop, uint64_t stride, const CellCopyArgs c,
                                                const uint32_t* cells, S* buf)
@@ -4947,6 +4950,50 @@ __global__ void __launch_bounds__(256) k_cells(void* pop, uint64_t stride, const
   }
 }
 
+// One thread a value, population blockIdx.y: 19 times the threads, for lists too
+// short to fill the chip otherwise and for scattered cells, bound by latency
+template <typename S, bool GATHER>
+__global__ void __launch_bounds__(256) k_cell_values(void* pop, uint64_t stride, const CellCopyArgs c,
+                                                     const uint32_t* cells, S* buf)
+{
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= c.n) {
+    return;
+  }
+  const uint32_t cell = cells[k];
+  if (cell >= c.count) {
+    return;
+  }
+  const int i = (int)blockIdx.y;
+  S* at = ring_at<S>(pop, stride, i, ring_slot(cell, c.shift[i], c.count));
+  buf += (size_t)i * c.n + k;
+  if constexpr (GATHER) {
+    *buf = *at;
+  } else {
+    *at = *buf;
+  }
+}
+
+// k_cells or k_cell_values?  us, one thread a value / a cell (gather, scatter):
+// 4096 random cells FP32 3.3 / 4.4, 3.4 / 5.4; a z plane of 128^3 6.3 / 8.5, 5.6 /
+// 6.4; 64000 consecutive cells 3.7 / 4.0, 3.8 / 4.4, but 130000 5.5 / 3.9, 5.6 /
+// 4.6 and 1 M 41 / 22, 42 / 20.  Of 256^3 every second cell FP32 521 / 344, 592 /
+// 734, FP16 448 / 185, 487 / 372; every fourth FP32 307 / 295, 614 / 650, FP16 239
+// / 144, 290 / 330; 1 M random ones FP32 343 / 397, 613 / 743; rows of 8 of 256
+// FP32 38 / 36, 43 / 37.  FP64, 200^3: half of the cells at random 338 / 400, 651
+// / 694, rows of 16 52 / 43, all 578 / 456, 560 / 621; 100^3 of it 77 / 49, 83 / 49
+bool per_cell(const olbgfx_lattice* L, const olbgfx_cell_list* list, bool gather)
+{
+  const double run = (double)list->n / list->runs, dense = (double)list->n / list->segments;
+  if (list->n < 100000) {
+    return false;
+  }
+  if (L->elem == 8) {
+    return gather ? run >= 16 : run >= 90 && list->n >= 300000 && list->n <= 4000000;
+  }
+  return run >= 8 || (gather && dense >= 12) || (L->elem == 2 && dense >= 28);
+}
+
 template <typename S>
 void cells_launch(olbgfx_lattice* L, const olbgfx_cell_list* list, void* buf, bool gather, hipStream_t s)
 {
@@ -4954,11 +5001,17 @@ void cells_launch(olbgfx_lattice* L, const olbgfx_cell_list* list, void* buf, bo
   for (int i = 0; i < Q; ++i) c.shift[i] = L->shift[i];
   c.count = L->count;
   c.n = list->n;
-  const dim3 grid((uint32_t)(((uint64_t)list->n + 255) / 256)), block(256);
-  if (gather) {
-    k_cells<S, true><<<grid, block, 0, s>>>(L->pop, L->stride, c, list->cells, (S*)buf);
+  const uint32_t blocks = (uint32_t)(((uint64_t)list->n + 255) / 256);
+  if (per_cell(L, list, gather)) {
+    if (gather) {
+      k_cells<S, true><<<blocks, 256, 0, s>>>(L->pop, L->stride, c, list->cells, (S*)buf);
+    } else {
+      k_cells<S, false><<<blocks, 256, 0, s>>>(L->pop, L->stride, c, list->cells, (S*)buf);
+    }
+  } else if (gather) {
+    k_cell_values<S, true><<<dim3(blocks, Q), 256, 0, s>>>(L->pop, L->stride, c, list->cells, (S*)buf);
   } else {
-    k_cells<S, false><<<grid, block, 0, s>>>(L->pop, L->stride, c, list->cells, (S*)buf);
+    k_cell_values<S, false><<<dim3(blocks, Q), 256, 0, s>>>(L->pop, L->stride, c, list->cells, (S*)buf);
   }
 }
 
@@ -5011,6 +5064,10 @@ olbgfx_status olbgfx_cell_list_create(const olbgfx_lattice* L, const uint32_t* c
   }
   list->n = n;
   list->count = L->count;
+  for (uint32_t k = 0; k < n; ++k) {
+    list->runs += k == 0 || cells[k] != cells[k - 1] + 1 ? 1 : 0;
+    list->segments += k == 0 || cells[k] / 64 != cells[k - 1] / 64 ? 1 : 0;
+  }
   if (n > 0) {
     if (device_alloc(&list->cells, sizeof(uint32_t) * n) != hipSuccess) {
       (void)hipGetLastError();
