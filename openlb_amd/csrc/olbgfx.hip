@@ -4343,9 +4343,12 @@ olbgfx_status ensemble_enqueue(olbgfx_ensemble* E, uint32_t steps, hipStream_t s
       all.ntiles = E->ntiles;
       all.member_end = groups.back().member_end;
       groups.assign(1, all);
-      if (!E->launch_given) {
+      uint64_t bytes = 0;
+      for (const olbgfx_lattice* L : E->members) bytes += (uint64_t)Q * L->stride * L->elem;
+      if (!E->launch_given && bytes >= (256ull << 20)) {
         // as in default_launch: all members FP32 1630 / 1552 us with 4 waves a
-        // SIMD, FP16 913 / 891 with 5
+        // SIMD, FP16 913 / 891 with 5; ensembles that the cache holds lose with a
+        // cap (4 cavities 64^3 FP32 32.3 / 34.7 us, FP16 22.1 / 23.6)
         lds = lds_for(E->block_threads, sizeof(S) == 4 ? 4 : (sizeof(S) == 2 ? 5 : 0));
       }
     }
