@@ -288,19 +288,21 @@ olbgfx_status olbgfx_get_statistics(olbgfx_lattice* lattice, double out[4]);
 /* FP64 conservation check over all colliding core cells, computed from the
  * stored populations: out = {nCells, sum (rho-1), sum j_x, sum j_y, sum j_z,
  * sum |u|^2, max |u|^2, 0}.  Replaces the thrust reductions of
- * core/platform/gpu/hip/statistics.hh:79-115.  Synchronises. */
+ * core/platform/gpu/hip/statistics.hh:79-115.  The first call allocates a
+ * workspace of 1/4 byte a cell, which the lattice keeps.  Calls on different
+ * lattices do not wait for each other.  Synchronises. */
 olbgfx_status olbgfx_reduce_moments(olbgfx_lattice* lattice, double out[8], void* stream);
 
 /* The same reduction for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  It runs the kernel of
  * olbgfx_reduce_moments into a fixed device array of the library (4 MiB per
- * device, held until the process ends) instead of a temporary allocation,
+ * device, held until the process ends) instead of the lattice's workspace,
  * and returns the same values bit for bit.  Lattices of more than 2^24 core
  * cells (65536 blocks of 256) are refused with OLBGFX_ERR_INVALID.  It calls
  * no hipMalloc or hipFree.  Calls within one process are serialised on a
- * lock, since every call on a device shares that device's array; the sums of
- * its rows are taken on the device.  Synchronises. */
+ * lock, since every call on a device shares that device's array; the lock is
+ * taken when the work of `stream` is done.  Synchronises. */
 olbgfx_status olbgfx_reduce_moments_noalloc(olbgfx_lattice* lattice, double out[8], void* stream);
 
 /* density and velocity of every padded cell through the momenta of its

@@ -1929,6 +1929,7 @@ namespace {
 // that device with the device current
 constexpr int kNoAllocMaxDevices = 64;
 double* g_noalloc_dev[kNoAllocMaxDevices] = {};
+double* g_noalloc_out = nullptr;  // pinned, the result of a call; allocated with the first lattice
 std::mutex g_noalloc_mutex;
 
 // caller holds g_noalloc_mutex
@@ -1975,7 +1976,11 @@ struct olbgfx_lattice {
   void* cell_rho = nullptr;
   void* cell_force = nullptr;
   double* stats_partial = nullptr;
-  double* moments_out = nullptr; // pinned host memory that the device writes (8 doubles)
+  // workspace of olbgfx_reduce_moments, from the first call on: the partials of
+  // its blocks (1/4 byte a cell) and pinned host memory that the device writes
+  double* moments_partial = nullptr;
+  double* moments_out = nullptr;
+  std::mutex moments_mutex;
   double* stats_out = nullptr;   // pinned host memory that the device writes (4 doubles)
   uint32_t stats_capacity = 0;
   bool stats_on = false;
@@ -3083,11 +3088,12 @@ olbgfx_status dispatch_storage(olbgfx_lattice* L, F&& f)
   }
 }
 
-// k_moments over all blocks and their sums, into out, under g_noalloc_mutex
-olbgfx_status moments(olbgfx_lattice* L, double* partial, uint32_t nb, double* out, hipStream_t s)
+// k_moments over all blocks and their sums, through partial and the pinned
+// result, into out.  The caller has waited for s and holds the lock of the two
+// workspaces, so a call never waits under a lock for the work of another.
+olbgfx_status moments(olbgfx_lattice* L, double* partial, uint32_t nb, double* result, double* out, hipStream_t s)
 {
   const olbgfx_lattice_desc& D = L->desc;
-  HIP_TRY(hipStreamSynchronize(s));
   if (sync_shifts(L) != OLBGFX_OK) {
     return OLBGFX_ERR_HIP;
   }
@@ -3102,15 +3108,15 @@ olbgfx_status moments(olbgfx_lattice* L, double* partial, uint32_t nb, double* o
     return st;
   }
   const uint32_t sums = (nb + kMomentsChunk - 1) / kMomentsChunk;
-  k_moments_sum<<<sums, 1024, 0, s>>>(partial, nb, kMomentsChunk, 1, sums > 1 ? nullptr : L->moments_out);
+  k_moments_sum<<<sums, 1024, 0, s>>>(partial, nb, kMomentsChunk, 1, sums > 1 ? nullptr : result);
   if (sums > 1) {
-    k_moments_sum<<<1, 1024, 0, s>>>(partial, sums, sums, kMomentsChunk, L->moments_out);
+    k_moments_sum<<<1, 1024, 0, s>>>(partial, sums, sums, kMomentsChunk, result);
   }
   HIP_TRY(hipGetLastError());
   if (hipStreamSynchronize(s) != hipSuccess) {
     return fail(OLBGFX_ERR_HIP, "moment reduction failed");
   }
-  std::memcpy(out, L->moments_out, 8 * sizeof(double));
+  std::memcpy(out, result, 8 * sizeof(double));
   return OLBGFX_OK;
 }
 
@@ -3437,9 +3443,13 @@ olbgfx_status olbgfx_lattice_create(const olbgfx_lattice_desc* desc, olbgfx_latt
   if (device_alloc(&L->pop, bytes) != hipSuccess) {
     return cleanup(fail(OLBGFX_ERR_NOMEM, "population allocation failed"));
   }
-  if (hipHostMalloc((void**)&L->moments_out, 8 * sizeof(double), hipHostMallocPortable) != hipSuccess) {
-    L->moments_out = nullptr;
-    return cleanup(fail(OLBGFX_ERR_NOMEM, "host allocation failed"));
+  {
+    std::lock_guard<std::mutex> lock(g_noalloc_mutex);
+    if (!g_noalloc_out &&
+        hipHostMalloc((void**)&g_noalloc_out, 8 * sizeof(double), hipHostMallocPortable) != hipSuccess) {
+      g_noalloc_out = nullptr;
+      return cleanup(fail(OLBGFX_ERR_NOMEM, "host allocation failed"));
+    }
   }
   if (hipMemset(L->pop, 0, bytes) != hipSuccess ||
       device_alloc(&L->mask, count) != hipSuccess || hipMemset(L->mask, 0, count) != hipSuccess ||
@@ -3477,6 +3487,7 @@ olbgfx_status olbgfx_lattice_destroy(olbgfx_lattice* L)
   hipFree(L->bzv_q);
   hipFree(L->bzv_v);
   hipFree(L->stats_partial);
+  hipFree(L->moments_partial);
   if (L->moments_out) {
     (void)hipHostFree(L->moments_out);
   }
@@ -3990,15 +4001,19 @@ olbgfx_status olbgfx_reduce_moments(olbgfx_lattice* L, double out[8], void* stre
   }
   const olbgfx_lattice_desc& D = L->desc;
   const uint64_t nb = ((uint64_t)D.nx * D.ny * D.nz + 255) / 256;
-  if (nb <= kNoAllocBlocks) {
-    return olbgfx_reduce_moments_noalloc(L, out, stream);
+  HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+  std::lock_guard<std::mutex> lock(L->moments_mutex);
+  if (!L->moments_out) {
+    if (hipHostMalloc((void**)&L->moments_out, 8 * sizeof(double), hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      L->moments_out = nullptr;
+      return fail(OLBGFX_ERR_NOMEM, "host allocation failed");
+    }
   }
-  std::lock_guard<std::mutex> lock(g_noalloc_mutex);
-  double* partial = nullptr;
-  HIP_TRY(device_alloc(&partial, 8 * sizeof(double) * (size_t)nb));
-  const olbgfx_status st = moments(L, partial, (uint32_t)nb, out, (hipStream_t)stream);
-  hipFree(partial);
-  return st;
+  if (!L->moments_partial) {
+    HIP_TRY(device_alloc(&L->moments_partial, 8 * sizeof(double) * (size_t)nb));
+  }
+  return moments(L, L->moments_partial, (uint32_t)nb, L->moments_out, out, (hipStream_t)stream);
 }
 
 olbgfx_status olbgfx_reduce_moments_noalloc(olbgfx_lattice* L, double out[8], void* stream)
@@ -4014,8 +4029,9 @@ olbgfx_status olbgfx_reduce_moments_noalloc(olbgfx_lattice* L, double out[8], vo
                 "olbgfx_reduce_moments_noalloc: the lattice has more than 16777216 core cells "
                 "(65536 blocks of 256), the size of its fixed device scratch; use olbgfx_reduce_moments");
   }
-  // one call at a time per process: the device scratch is shared by every
-  // lattice, and a lattice has one place for the result
+  // one call at a time per process: the device scratch and the place of the
+  // result are shared by every lattice
+  HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
   std::lock_guard<std::mutex> lock(g_noalloc_mutex);
   double* partial = nullptr;
   if (noalloc_scratch(&partial) != OLBGFX_OK) {
@@ -4023,7 +4039,7 @@ olbgfx_status olbgfx_reduce_moments_noalloc(olbgfx_lattice* L, double out[8], vo
   }
   // k_moments writes all 8 slots of every block it runs, so nothing left in
   // the scratch by an earlier call is read
-  return moments(L, partial, (uint32_t)nb, out, (hipStream_t)stream);
+  return moments(L, partial, (uint32_t)nb, g_noalloc_out, out, (hipStream_t)stream);
 }
 
 olbgfx_status olbgfx_compute_rho_u(olbgfx_lattice* L, int32_t vt, void* rho, void* u)
