@@ -450,11 +450,15 @@ olbgfx_status olbgfx_device_buffer_destroy(void* device_buffer);
  *
  * Lattices: first every (block_threads x waves_per_simd) pair with the
  * default block order, then every block order with the three fastest pairs.
- * Ensembles: first every (block_threads x waves_per_simd x tiles_per_block)
- * with one group, then every block order with the three fastest, then every
- * (group_bytes x steps_per_group x ticket) with the best launch.  A list with n == 0 takes the built-in candidates; a null
- * `space` takes them all.  Each trial runs one untimed step (steps_per_group
- * for schedules) and then `steps` timed steps (ensembles: at least 8).
+ * Ensembles: first every (group_bytes x steps_per_group x ticket) with the
+ * first launch of the lists, then every (block_threads x waves_per_simd x
+ * tiles_per_block) in the fastest schedule, then every block order with the
+ * three fastest; the pick has to beat what the ensemble does until it is set
+ * (where the lists allow that: 200 MiB, 1024 steps, 256 threads, no cap), which
+ * is kept otherwise, and which picking it restores with its rules by call
+ * length.  A list with n == 0 takes the built-in candidates; a null `space`
+ * takes them all.  Each trial runs one untimed step (up to 8 for schedules) and
+ * then `steps` timed steps (ensembles: at least 32, in one call).
  *
  * `cache_path` (may be null) names a text file of earlier choices keyed by
  * extent, padding, periodicity, storage and the dynamics mix (ensembles: by

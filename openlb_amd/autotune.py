@@ -3,8 +3,8 @@ olbgfx_autotune_ensemble).
 
 For a lattice the library sweeps threads per block and an occupancy cap
 (waves per SIMD, enforced by an LDS reservation), then the order in which
-blocks visit the cells; for an ensemble the tiles each persistent block walks
-and the group schedule.  Every candidate is timed with HIP events on the
+blocks visit the cells; for an ensemble the group schedule, the launch shape
+and the tiles each persistent block walks.  Every candidate is timed with HIP events on the
 lattice itself, the fastest is applied, and the populations, offsets and
 statistics are put back as they were, so tuning does not advance the
 simulation.  Choices are cached in a text file keyed by shape, storage and
@@ -108,9 +108,9 @@ def tune_lattice(lat, steps: int = 4, stream=None, use_cache: bool = True,
 
 def tune_ensemble(ens, steps: int = 4, stream=None, use_cache: bool = True, blocks=None, waves=None,
                   tiles=None, orders=None, group_bytes=None, steps_per_group=None, tickets=None) -> dict:
-    """pick (block_threads, waves_per_simd, tiles_per_block), then the block
-    order, then the group schedule (group_bytes, steps_per_group, ticket), for
-    an ensemble"""
+    """pick the group schedule (group_bytes, steps_per_group, ticket), then
+    (block_threads, waves_per_simd, tiles_per_block) inside it, then the block
+    order, for an ensemble; what it does untuned stays if no pick beats it"""
     res = TuneResult()
     sp = _space(blocks=blocks, waves=waves, tiles=tiles, orders=orders, group_bytes=group_bytes,
                 steps_per_group=steps_per_group, tickets=tickets)

@@ -5253,7 +5253,8 @@ std::string tune_key(const olbgfx_ensemble* E)
     h = fnv1a(h, k.data(), k.size());
   }
   char buf[96];
-  std::snprintf(buf, sizeof(buf), "ensemble:%zu:s%d:%016llx", E->members.size(), E->storage,
+  // 2: picks of trials that the untuned schedule took part in
+  std::snprintf(buf, sizeof(buf), "ensemble2:%zu:s%d:%016llx", E->members.size(), E->storage,
                 (unsigned long long)h);
   return buf;
 }
@@ -5328,6 +5329,19 @@ std::vector<V> choices(uint32_t n, const V (&given)[N], const V (&defaults)[M])
     return std::vector<V>(defaults, defaults + M);
   }
   return std::vector<V>(given, given + std::min<size_t>(n, N));
+}
+
+template <typename V>
+bool allowed(const std::vector<V>& list, V value)
+{
+  return std::find(list.begin(), list.end(), value) != list.end();
+}
+
+bool same_choice(const olbgfx_tune_trial& a, const olbgfx_tune_trial& b)
+{
+  return a.block_threads == b.block_threads && a.waves_per_simd == b.waves_per_simd &&
+         a.block_order == b.block_order && a.tiles_per_block == b.tiles_per_block && a.group_bytes == b.group_bytes &&
+         a.steps_per_group == b.steps_per_group && a.ticket == b.ticket;
 }
 
 struct Trials {
@@ -5470,11 +5484,11 @@ olbgfx_status olbgfx_autotune_ensemble(olbgfx_ensemble* E, uint32_t steps, const
   if (!E || E->members.empty()) {
     return fail(OLBGFX_ERR_INVALID, "null or empty ensemble");
   }
-  static const uint32_t kBlocks[] = {128, 256};
+  static const uint32_t kBlocks[] = {256, 128};
   static const uint32_t kWaves[] = {0, 3, 4, 5};
   static const uint32_t kTiles[] = {1, 2, 4};
-  static const uint64_t kGroups[] = {0, 160ull << 20, kGroupBytes};
-  static const uint32_t kPerGroup[] = {1, 8, 64};
+  static const uint64_t kGroups[] = {kGroupBytes, 160ull << 20, 0};
+  static const uint32_t kPerGroup[] = {1024, 8, 1};
   static const int32_t kTickets[] = {0, 1};
   const olbgfx_tune_space none{};
   const olbgfx_tune_space& sp = space ? *space : none;
@@ -5489,10 +5503,24 @@ olbgfx_status olbgfx_autotune_ensemble(olbgfx_ensemble* E, uint32_t steps, const
   const std::string key = tune_key(E);
   Trials tr;
   olbgfx_tune_trial best{};
+  // what an ensemble does until it is set: a pick like any other, which stands
+  // for the rules by call length too
+  const olbgfx_tune_trial untuned = [] {
+    olbgfx_tune_trial t{};
+    t.block_threads = 256;
+    t.block_order = -1;
+    t.tiles_per_block = 1;
+    t.group_bytes = kGroupBytes;
+    t.steps_per_group = 1024;
+    return t;
+  }();
   auto apply = [&](const olbgfx_tune_trial& t) -> olbgfx_status {
     olbgfx_status r = olbgfx_ensemble_set_launch(E, t.block_threads, t.waves_per_simd, t.tiles_per_block);
     if (r == OLBGFX_OK) r = olbgfx_ensemble_set_block_order(E, t.block_order);
     if (r == OLBGFX_OK) r = olbgfx_ensemble_set_schedule(E, t.group_bytes, t.steps_per_group, t.ticket);
+    if (r == OLBGFX_OK && same_choice(t, untuned)) {
+      E->launch_given = E->schedule_given = false;
+    }
     return r;
   };
   if (cache_lookup(cache_path, key, best)) {
@@ -5503,64 +5531,93 @@ olbgfx_status olbgfx_autotune_ensemble(olbgfx_ensemble* E, uint32_t steps, const
     return st;
   }
   hipStream_t s = (hipStream_t)stream;
-  const uint32_t span = std::max(8u, steps);
+  // long enough for groups that stay for 8 steps and for all of a call to differ
+  const uint32_t span = std::max(32u, steps);
   std::vector<SavedState> saved(E->members.size());
   olbgfx_status st = OLBGFX_OK;
   for (size_t k = 0; k < E->members.size() && st == OLBGFX_OK; ++k) {
     st = save_state(E->members[k], s, saved[k]);
   }
-  auto trial = [&](const olbgfx_tune_trial& cand) -> olbgfx_status {
+  auto timed = [&](const olbgfx_tune_trial& cand, double& ms_per_step) -> olbgfx_status {
     olbgfx_status r = apply(cand);
-    if (r == OLBGFX_OK) r = olbgfx_ensemble_step(E, cand.steps_per_group, stream);
+    if (r == OLBGFX_OK) r = olbgfx_ensemble_step(E, std::min(cand.steps_per_group, 8u), stream);
     float ms = 0;
     if (r == OLBGFX_OK) r = olbgfx_ensemble_time(E, 0, span, stream, &ms);
+    ms_per_step = (double)ms / span;
+    return r;
+  };
+  auto trial = [&](olbgfx_tune_trial t) -> olbgfx_status {
+    const olbgfx_status r = timed(t, t.ms_per_step);
     if (r == OLBGFX_OK) {
-      olbgfx_tune_trial t = cand;
-      t.ms_per_step = (double)ms / span;
       tr.add(t);
     }
     return r;
   };
-  for (size_t i = 0; i < blocks.size() && st == OLBGFX_OK; ++i) {
-    for (size_t j = 0; j < waves.size() && st == OLBGFX_OK; ++j) {
-      for (size_t k = 0; k < tiles.size() && st == OLBGFX_OK; ++k) {
-        olbgfx_tune_trial c{};
-        c.block_threads = blocks[i];
-        c.waves_per_simd = waves[j];
-        c.block_order = -1;
-        c.tiles_per_block = tiles[k];
-        c.group_bytes = 0;
-        c.steps_per_group = 1;
-        c.ticket = 0;
-        st = trial(c);
-      }
-    }
-  }
-  const std::vector<olbgfx_tune_trial> shapes = fastest(tr.all, 3);
-  for (size_t m = 0; m < shapes.size() && st == OLBGFX_OK; ++m) {
-    for (size_t k = 0; k < orders.size() && st == OLBGFX_OK; ++k) {
-      if (orders[k] != -1) {
-        olbgfx_tune_trial c = shapes[m];
-        c.block_order = orders[k];
+  // the schedule first, then the launch inside the fastest one
+  olbgfx_tune_trial base{};
+  base.block_threads = blocks[0];
+  base.waves_per_simd = waves[0];
+  base.block_order = -1;
+  base.tiles_per_block = tiles[0];
+  for (size_t i = 0; i < groups.size() && st == OLBGFX_OK; ++i) {
+    for (size_t j = 0; j < per_group.size() && st == OLBGFX_OK; ++j) {
+      for (size_t k = 0; k < tickets.size() && st == OLBGFX_OK; ++k) {
+        olbgfx_tune_trial c = base;
+        c.group_bytes = groups[i];
+        c.steps_per_group = per_group[j];
+        c.ticket = tickets[k] ? 1 : 0;
         st = trial(c);
       }
     }
   }
   if (st == OLBGFX_OK && !tr.all.empty()) {
     const olbgfx_tune_trial first = tr.all[tr.best];
-    for (size_t i = 0; i < groups.size() && st == OLBGFX_OK; ++i) {
-      for (size_t j = 0; j < per_group.size() && st == OLBGFX_OK; ++j) {
-        for (size_t k = 0; k < tickets.size() && st == OLBGFX_OK; ++k) {
-          if (groups[i] == 0 && per_group[j] == 1 && tickets[k] == 0) {
-            continue;  // the launch phase already timed this schedule
-          }
+    std::vector<olbgfx_tune_trial> shapes(1, first);
+    for (size_t i = 0; i < blocks.size() && st == OLBGFX_OK; ++i) {
+      for (size_t j = 0; j < waves.size() && st == OLBGFX_OK; ++j) {
+        for (size_t k = 0; k < tiles.size() && st == OLBGFX_OK; ++k) {
           olbgfx_tune_trial c = first;
-          c.group_bytes = groups[i];
-          c.steps_per_group = per_group[j];
-          c.ticket = tickets[k] ? 1 : 0;
+          c.block_threads = blocks[i];
+          c.waves_per_simd = waves[j];
+          c.tiles_per_block = tiles[k];
+          if (!same_choice(c, first)) {
+            st = trial(c);
+            shapes.push_back(tr.all.back());
+          }
+        }
+      }
+    }
+    shapes = fastest(shapes, 3);
+    for (size_t m = 0; m < shapes.size() && st == OLBGFX_OK; ++m) {
+      for (size_t k = 0; k < orders.size() && st == OLBGFX_OK; ++k) {
+        if (orders[k] != -1) {
+          olbgfx_tune_trial c = shapes[m];
+          c.block_order = orders[k];
           st = trial(c);
         }
       }
+    }
+  }
+  // A pick has to beat what the ensemble does untuned, in turns, by more than
+  // they scatter, if the caller's lists allow that.
+  if (st == OLBGFX_OK && !tr.all.empty() && !same_choice(tr.all[tr.best], untuned) &&
+      allowed(blocks, untuned.block_threads) && allowed(waves, untuned.waves_per_simd) &&
+      allowed(tiles, untuned.tiles_per_block) && allowed(orders, untuned.block_order) &&
+      allowed(groups, untuned.group_bytes) && allowed(per_group, untuned.steps_per_group) &&
+      allowed(tickets, untuned.ticket)) {
+    double pick = 1e30, plain = 1e30;
+    for (int k = 0; k < 3 && st == OLBGFX_OK; ++k) {
+      double ms = 0;
+      st = timed(tr.all[tr.best], ms);
+      pick = std::min(pick, ms);
+      if (st == OLBGFX_OK) st = timed(untuned, ms);
+      plain = std::min(plain, ms);
+    }
+    if (st == OLBGFX_OK && pick > 0.99 * plain) {
+      olbgfx_tune_trial t = untuned;
+      t.ms_per_step = plain;
+      tr.all.push_back(t);
+      tr.best = tr.all.size() - 1;
     }
   }
   const std::string err = st == OLBGFX_OK ? std::string() : g_error;
