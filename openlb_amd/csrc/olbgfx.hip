@@ -2618,18 +2618,30 @@ void launch_pair_form(bool src_ring, bool dst_ring, dim3 grid, hipStream_t strea
 }
 
 template <typename S, uint32_t NT>
-void launch_pair_mode(int mode, bool periodic, bool src_ring, bool dst_ring, dim3 grid, hipStream_t stream,
+bool launch_pair_mode(int mode, bool periodic, bool src_ring, bool dst_ring, dim3 grid, hipStream_t stream,
                       const PairArgs<typename Storage<S>::A>& p)
 {
+  // the forms that pair_threads chooses: 512 threads in 4-byte storage for BGK
+  // only, 1024 in BF16 for all but BGK
+  constexpr bool small = sizeof(S) == 4 && NT == 512;
   if (periodic) {
     switch (mode) {
     case OLBGFX_BGK:
-      return launch_pair_form<S, NT, OLBGFX_BGK, true>(src_ring, dst_ring, grid, stream, p);
+      if constexpr (NT == 512 || !std::is_same_v<S, bf16_t>) {
+        launch_pair_form<S, NT, OLBGFX_BGK, true>(src_ring, dst_ring, grid, stream, p);
+        return true;
+      }
+      break;
     case OLBGFX_FORCED_TRT:
-      return launch_pair_form<S, NT, OLBGFX_FORCED_TRT, true>(src_ring, dst_ring, grid, stream, p);
+      if constexpr (!small) {
+        launch_pair_form<S, NT, OLBGFX_FORCED_TRT, true>(src_ring, dst_ring, grid, stream, p);
+        return true;
+      }
+      break;
     case OLBGFX_SMAGORINSKY_BGK:
-      if constexpr (sizeof(S) > 2) {
-        return launch_pair_form<S, NT, OLBGFX_SMAGORINSKY_BGK, true>(src_ring, dst_ring, grid, stream, p);
+      if constexpr (sizeof(S) > 2 && !small) {
+        launch_pair_form<S, NT, OLBGFX_SMAGORINSKY_BGK, true>(src_ring, dst_ring, grid, stream, p);
+        return true;
       }
       break;
     default:
@@ -2651,7 +2663,9 @@ void launch_pair_mode(int mode, bool periodic, bool src_ring, bool dst_ring, dim
     } else {
       masked(std::false_type{});
     }
+    return true;
   }
+  return false;
 }
 
 // two steps from src to dst; shift: the source offsets, dshift those of the
@@ -2694,12 +2708,14 @@ olbgfx_status launch_pair(olbgfx_lattice* L, const StepArgs<typename Storage<S>:
   p.nwork = plan.nwork;
   p.per_xcd = (p.nwork + 7) / 8;
   const dim3 grid(8 * p.per_xcd);
-  if constexpr (sizeof(S) == 8) {
-    launch_pair_mode<S, 512>(mode, periodic, src_ring, dst_ring, grid, stream, p);
-  } else if (plan.threads == 512) {
-    launch_pair_mode<S, 512>(mode, periodic, src_ring, dst_ring, grid, stream, p);
-  } else {
-    launch_pair_mode<S, 1024>(mode, periodic, src_ring, dst_ring, grid, stream, p);
+  bool launched = false;
+  if (sizeof(S) == 8 || plan.threads == 512) {
+    launched = launch_pair_mode<S, 512>(mode, periodic, src_ring, dst_ring, grid, stream, p);
+  } else if constexpr (sizeof(S) < 8) {
+    launched = launch_pair_mode<S, 1024>(mode, periodic, src_ring, dst_ring, grid, stream, p);
+  }
+  if (!launched) {
+    return fail(OLBGFX_ERR_HIP, "no kernel for two steps a pass of this form");
   }
   HIP_TRY(hipGetLastError());
   return OLBGFX_OK;
