@@ -2138,22 +2138,29 @@ uint32_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
 // keep the cells in flight together.  us a step, no cap and contiguous parts
 // against these: 512^3 FP32 4350 / 3960, FP16 2228 / 2076; slab 64x512x512 FP32
 // 538 / 497, FP16 279 / 263; 256^3 FP32 550 / 509, cavity 552 / 509, FP64 1051
-// / 1018; porous channel FP16 125 / 120.  Between 256 MiB and 1 GiB contiguous
-// parts stay better in 4-byte storage (40x300x400 capped: 138 against 144, 150
-// without the cap), and below 224 MiB the cache serves them best (160^3 FP16
-// 47 against 49, cavity 33^3 FP32 4.8 against 5.3).  Velocity and pressure
-// boundaries hide their chains of loads behind other waves, so steps with them
-// take no cap (LocalVelocity cavity FP32, capped / uncapped: 150^3 162 / 141,
-// 200^3 331 / 314, 240^3 560 / 526).
+// / 1018.  Between 256 MiB and 1 GiB contiguous parts stay better in 4-byte
+// storage (40x300x400 capped: 138 against 144, 150 without the cap), and below
+// 256 MiB the cache serves them best (160^3 FP16 47 against 49, 446x87x163 BF16
+// of 238 MiB 65 against 70, cavity 33^3 FP32 4.8 against 5.3).
+// The cap is for kernels with registers for more than 4 waves that wait for
+// memory alone: BGK, TRT and Smagorinsky on 60 random boxes of 256 to 480 MiB
+// 0.89 to 0.99 of the time without, but forced kinds 0.98 to 1.03, masked cells
+// on periodic lattices up to 1.06 (others 0.95 to 1.05, from 512 MiB 0.95 to
+// 1.00), and velocity and pressure boundaries, which hide their chains of loads behind other waves,
+// more (LocalVelocity cavity, 150^3 162 against 141 us, 200^3 331 / 314).
 void default_launch(const olbgfx_lattice* L, uint32_t& lds, int32_t& order)
 {
   const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
-  const bool capped = L->elem == 4 && mib >= 256 && !L->boundary_kinds;
+  const int32_t* P = L->desc.periodic;
+  const int kind = L->uniform_id >= 0 ? L->table[L->uniform_id].kind : -1;
+  const bool waits = kind == OLBGFX_BGK || kind == OLBGFX_TRT || kind == OLBGFX_SMAGORINSKY_BGK ||
+                     (kind < 0 && !L->boundary_kinds && !(P[0] && P[1] && P[2]) && mib >= 512);
+  const bool capped = L->elem == 4 && mib >= 256 && waits;
   lds = L->launch_given ? L->lds_reserve : (capped ? lds_for(L->block_threads, 4) : 0);
   if (L->order_given) {
     order = L->xcd_run_log2;
   } else if (L->elem == 2) {
-    order = mib >= 224 ? 3 : -1;
+    order = mib >= 256 ? 3 : -1;
   } else {
     order = mib >= 1024 ? 4 : -1;
   }

@@ -53,7 +53,8 @@ BULK = {"bgk": Dynamics(BGK, omega=1 / 0.6), "forced_trt": Dynamics(FORCED_TRT, 
 
 
 def _box(storage, kind, extent, padding):
-    """a uniform periodic box, or one of BGK closed by bounce-back cells"""
+    """a uniform periodic box, one of BGK closed by bounce-back cells, or a
+    periodic one of ForcedTRT with oblique walls"""
     lat = Lattice(extent, padding, (kind != "closed",) * 3, storage)
     mask = np.zeros(tuple(n + 2 * padding for n in extent), dtype=np.uint8)
     mask[tuple(slice(padding, -padding) for _ in range(3))] = 1
@@ -62,8 +63,36 @@ def _box(storage, kind, extent, padding):
         lat.set_dynamics(2, Dynamics(BOUNCE_BACK))
         mask[mask == 1] = 2
         mask[tuple(slice(padding + 1, -padding - 1) for _ in range(3))] = 1
+    if kind == "porous":
+        lat.set_dynamics(1, BULK["forced_trt"])
+        lat.set_dynamics(2, Dynamics(BOUNCE_BACK))
+        x, y, z = (np.arange(n) for n in mask.shape)
+        mask[((x[:, None, None] + y[:, None] + z) % 23 < 7) & (mask > 0)] = 2
     lat.set_dynamics_mask(mask)
     return lat
+
+
+@pytest.mark.parametrize("storage,kind,extent", [("bf16", "bgk", (446, 87, 163)), ("f16", "bgk", (204, 125, 259)),
+                                                 ("f32", "porous", (116, 139, 227))])
+def test_single_steps_near_the_cache_size(storage, kind, extent):
+    """turns on short runs of blocks, which the cache does without (1.08 and
+    1.09), and a cap for masked cells of a periodic lattice (1.06)"""
+    print(f"[launch defaults] {storage} {kind} {extent} single steps", flush=True)
+    lats = [_box(storage, kind, extent, 1) for _ in range(2)]
+    lats[1].set_launch(256, 0)
+    lats[1].set_block_order(-1)
+
+    def steps(lat):
+        for _ in range(40):
+            lat.collide_and_stream(1)
+        lat.synchronize()
+
+    for lat in lats:
+        steps(lat)
+    default, plain = least([lambda: steps(lats[0]), lambda: steps(lats[1])])
+    for lat in lats:
+        lat.close()
+    assert default <= 1.035 * plain
 
 
 # runs that took 1.08 to 1.2 of the single steps' time two steps a pass
