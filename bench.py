@@ -84,6 +84,7 @@ def time_storage(torch, size, storage, steps, warmup, block, tune=True):
     torch.cuda.synchronize()
 
     # whole-job timing: K steps between two synchronisations
+    before = lat.get_two_step()[1]
     t0 = time.perf_counter()
     start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     start.record(stream)
@@ -92,9 +93,10 @@ def time_storage(torch, size, storage, steps, warmup, block, tune=True):
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     ms_total = start.elapsed_time(stop)
+    in_pairs = lat.get_two_step()[1] - before
 
-    # per-launch kernel duration: HIP events around single steps on the stream
-    # the kernel is launched on
+    # duration of single steps (one kernel each), which a run does not take:
+    # HIP events around them on the stream they are launched on
     durs = []
     for _ in range(min(steps, 20)):
         a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -109,6 +111,10 @@ def time_storage(torch, size, storage, steps, warmup, block, tune=True):
     cells = size ** 3
     return {
         "ms_per_step": ms_total / steps,
+        "ms_total": ms_total,
+        "steps_two_a_pass": in_pairs,
+        # passes over the populations: one for two steps, or one a step
+        "passes": steps - in_pairs // 2,
         "wall_s": wall,
         "glups": cells * steps / (ms_total * 1e-3) / 1e9,
         "kernel_ms": kernel_ms,
@@ -399,12 +405,25 @@ def cpu_baseline(size, steps):
             "sample": f"C restatement (OpenMP) BGK TGV {size}^3 FP32, {steps} steps after 2 warm-up"}
 
 
-def load_traffic(storage):
-    path = os.path.join(ROOT, "profiles", f"traffic_step_{storage}_tgv512.json")
+def load_traffic(kernel, storage):
+    """(kernel, bytes a launch) as counted at 512^3, of the "pair" or "step" kernel"""
+    path = os.path.join(ROOT, "profiles", f"traffic_{kernel}_{storage}_tgv512.json")
     if os.path.exists(path):
         with open(path) as fh:
-            return json.load(fh).get("bytes_per_launch")
-    return None
+            d = json.load(fh)
+            return d["kernel"], d["bytes_per_launch"]
+    return None, None
+
+
+def rooflines(res, cells):
+    """algorithmic bytes (the populations read and written once a pass) over
+    time, of the timed run and of single steps, for each storage"""
+    out = {}
+    for st, v in res.items():
+        run = v["bytes_per_cell"] * cells * v["passes"] / (v["ms_total"] * 1e-3) / 1e9
+        single = v["bytes_per_cell"] * cells / (v["kernel_ms"] * 1e-3) / 1e9
+        out[st] = (run, single)
+    return out
 
 
 def main():
@@ -479,9 +498,14 @@ def main():
         print("# OpenLB cavity3dBenchmark on GPU_GFX950, RESOLUTION 100, 1000 steps: "
               + ", ".join(f"{k} {v['mlups']:.0f} MLUPs" for k, v in cases.items()), file=sys.stderr)
     cells = args.size ** 3
-    alg_bytes = head["bytes_per_cell"] * cells
-    achieved = alg_bytes / (head["kernel_ms"] * 1e-3) / 1e9
-    traffic = load_traffic(head_storage)
+    reached = rooflines(res, cells)
+    achieved, single = reached[head_storage]
+    kernel = "pair" if head["steps_two_a_pass"] else "step"
+    name, traffic = load_traffic(kernel, head_storage)
+    single_name, single_traffic = load_traffic("step", head_storage)
+    # of the kernel that the timed run spends its time in: one launch takes two
+    # steps where the library runs them so, and then moves per pass what a single
+    # step moves (`bytes_per_cell`)
     roofline = {
         "bound": "hbm",
         "achieved": round(achieved, 1),
@@ -489,16 +513,20 @@ def main():
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBPS, 4),
         "traffic": traffic,
-        "kernel": f"step_kernel<{head_storage}, BGK>",
+        "kernel": name or f"{kernel}_kernel<{head_storage}, BGK>",
         "bytes_per_cell": head["bytes_per_cell"],
+        "steps_two_a_pass": head["steps_two_a_pass"],
+        "single_step": {"kernel": single_name or f"step_kernel<{head_storage}, BGK>", "achieved": round(single, 1),
+                        "frac": round(single / HBM_PEAK_GBPS, 4), "traffic": single_traffic},
     }
     if probes:
         p = probes[head_storage]
-        roofline.update({
-            "measured_copy_GBps": p["copy"],
-            "frac_of_measured_copy": round(achieved / p["copy"], 4),
+        roofline.update({"measured_copy_GBps": p["copy"], "frac_of_measured_copy": round(achieved / p["copy"], 4)})
+        # the in-place rings are the pattern of single steps
+        roofline["single_step"].update({
+            "frac_of_measured_copy": round(single / p["copy"], 4),
             "pattern_ceiling_GBps": p["ring_inplace"],
-            "frac_of_pattern_ceiling": round(achieved / p["ring_inplace"], 4),
+            "frac_of_pattern_ceiling": round(single / p["ring_inplace"], 4),
         })
     base = None if args.no_cpu_baseline else cpu_baseline(args.cpu_size, args.cpu_steps)
     line = {
@@ -517,9 +545,9 @@ def main():
         "config": {"workload": f"taylor_green_d3q19_bgk_{args.size}^3", "cells": cells, "tau": 0.56,
                    "u0": 0.04, "storage": head_storage, "parallelism": "single GPU"},
         "storage_glups": {k: round(v["glups"], 3) for k, v in res.items()},
-        "storage_launch": {k: v["launch"] for k, v in res.items()},
-        "storage_hbm_frac": {k: round(v["bytes_per_cell"] * cells / (v["kernel_ms"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)
-                             for k, v in res.items()},
+        "storage_hbm_frac": {k: round(v[0] / HBM_PEAK_GBPS, 4) for k, v in reached.items()},
+        "single_step": {k: {"ms": round(v["kernel_ms"], 4), "glups": round(v["kernel_glups"], 3), "launch": v["launch"],
+                            "hbm_frac": round(reached[k][1] / HBM_PEAK_GBPS, 4)} for k, v in res.items()},
         "fp16_over_fp32": round(res["f16"]["glups"] / res["f32"]["glups"], 3) if "f16" in res and "f32" in res else None,
         "ensemble": {k: {kk: (round(vv, 3) if isinstance(vv, float) else vv) for kk, vv in v.items()}
                      for k, v in ens.items()},

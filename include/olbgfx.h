@@ -251,8 +251,10 @@ olbgfx_status olbgfx_set_populations(olbgfx_lattice* lattice, int32_t value_type
  * where that is faster (by size, kind and number of steps), on lattices that are periodic along every axis or
  * along none, without velocity-boundary or Bouzidi cells and without an
  * in-flight limit.  Results do not change, in any storage, however the steps
- * are split into calls, except that the padding cells of a periodic lattice
- * then hold no population but those that enter or left the core.  The first
+ * are split into calls.  Of the padding cells of a periodic lattice only the
+ * populations that entered or left the core are defined after such a run; the
+ * others, and with them the density and velocity of padding cells that have
+ * dynamics and the padding in a checkpoint, carry no meaning.  The first
  * such run allocates a second set of populations, which the lattice keeps
  * (olbgfx_set_two_step).  A stream under capture takes single steps. */
 olbgfx_status olbgfx_collide_and_stream(olbgfx_lattice* lattice, uint32_t steps, void* stream);
