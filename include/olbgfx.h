@@ -319,7 +319,7 @@ olbgfx_status olbgfx_compute_rho_u(olbgfx_lattice* lattice, int32_t value_type, 
  * threads per block of the step kernel (64..256, multiple of 64; 0 = 256) and
  * an occupancy cap in waves per SIMD (1..8; 0 = as many as registers allow),
  * enforced by reserving LDS per block.  Until this is called, 256 threads and
- * a cap chosen by the size of the lattice.  Used by the autotuner; no reference
+ * a cap chosen by the size and the dynamics of the lattice.  Used by the autotuner; no reference
  * counterpart (the reference fixes 64-thread blocks,
  * core/platform/gpu/hip/operator.hh:426-433). */
 olbgfx_status olbgfx_set_launch(olbgfx_lattice* lattice, uint32_t block_threads,
@@ -331,6 +331,10 @@ olbgfx_status olbgfx_set_launch(olbgfx_lattice* lattice, uint32_t block_threads,
  * size of the lattice.  Results do not depend
  * on it.  Used by the autotuner; no reference counterpart. */
 olbgfx_status olbgfx_set_block_order(olbgfx_lattice* lattice, int32_t xcd_run_log2);
+
+/* what single steps are launched with now, set or chosen */
+olbgfx_status olbgfx_get_launch(olbgfx_lattice* lattice, uint32_t* block_threads,
+                                uint32_t* waves_per_simd, int32_t* xcd_run_log2);
 
 /* ---- ensembles of independent lattices ------------------------------------
  * A batch of lattices (same storage type, any extents and dynamics) advanced

@@ -100,6 +100,7 @@ def library() -> ctypes.CDLL:
         "olbgfx_device_count": [ctypes.POINTER(i32)],
         "olbgfx_set_split": [vp, i32],
         "olbgfx_get_split": [vp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_uint32)],
+        "olbgfx_get_launch": [vp, ctypes.POINTER(u32), ctypes.POINTER(u32), ctypes.POINTER(i32)],
         "olbgfx_set_two_step": [vp, ctypes.c_uint64],
         "olbgfx_get_two_step": [vp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)],
         "olbgfx_probe_bandwidth": [ctypes.POINTER(_LatticeDesc), i32, u32, i32, u32, vp,
@@ -367,6 +368,13 @@ class Lattice:
         """threads per block (64..256) and an occupancy cap in waves per SIMD
         (0 = no cap)"""
         _check(library().olbgfx_set_launch(self._h, int(block_threads), int(waves_per_simd)))
+
+    def get_launch(self) -> tuple:
+        """(block_threads, waves_per_simd, xcd_run_log2) of single steps, set
+        or chosen by size and dynamics"""
+        block, waves, order = ctypes.c_uint32(), ctypes.c_uint32(), ctypes.c_int32()
+        _check(library().olbgfx_get_launch(self._h, ctypes.byref(block), ctypes.byref(waves), ctypes.byref(order)))
+        return block.value, waves.value, order.value
 
     def set_split(self, on: bool = True) -> None:
         """split steps (the dominant dynamics' own kernel plus a masked

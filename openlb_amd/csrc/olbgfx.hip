@@ -1987,7 +1987,7 @@ struct olbgfx_lattice {
   bool stats_valid = false;
   int32_t uniform_id = 0;     // all cells start with id 0 = NoDynamics
   uint32_t block_threads = 256;
-  uint32_t lds_reserve = 0;    // dynamic LDS per block that limits occupancy
+  uint32_t waves = 0;          // occupancy cap in waves per SIMD (0: none)
   int32_t xcd_run_log2 = -1;   // block order of the step kernel (olbgfx_set_block_order)
   bool launch_given = false, order_given = false;  // else chosen by size (default_launch)
   // LocalVelocity boundaries: discrete normals, and the cells whose
@@ -2148,7 +2148,7 @@ uint32_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
 // on periodic lattices up to 1.06 (others 0.95 to 1.05, from 512 MiB 0.95 to
 // 1.00), and velocity and pressure boundaries, which hide their chains of loads behind other waves,
 // more (LocalVelocity cavity, 150^3 162 against 141 us, 200^3 331 / 314).
-void default_launch(const olbgfx_lattice* L, uint32_t& lds, int32_t& order)
+void default_launch(const olbgfx_lattice* L, uint32_t& waves, int32_t& order)
 {
   const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
   const int32_t* P = L->desc.periodic;
@@ -2156,7 +2156,7 @@ void default_launch(const olbgfx_lattice* L, uint32_t& lds, int32_t& order)
   const bool waits = kind == OLBGFX_BGK || kind == OLBGFX_TRT || kind == OLBGFX_SMAGORINSKY_BGK ||
                      (kind < 0 && !L->boundary_kinds && !(P[0] && P[1] && P[2]) && mib >= 512);
   const bool capped = L->elem == 4 && mib >= 256 && waits;
-  lds = L->launch_given ? L->lds_reserve : (capped ? lds_for(L->block_threads, 4) : 0);
+  waves = L->launch_given ? L->waves : (capped ? 4 : 0);
   if (L->order_given) {
     order = L->xcd_run_log2;
   } else if (L->elem == 2) {
@@ -2190,8 +2190,8 @@ olbgfx_status fill_args(olbgfx_lattice* L, StepArgs<A>& a, bool device_shifts)
   a.ncore = (uint32_t)D.nx * a.nyz;
   a.nblocks = (a.ncore + L->block_threads - 1) / L->block_threads;
   a.blocks_per_xcd = (a.nblocks + 7) / 8;
-  uint32_t lds = 0;
-  default_launch(L, lds, a.xcd_run_log2);
+  uint32_t waves = 0;
+  default_launch(L, waves, a.xcd_run_log2);
   if (a.xcd_run_log2 >= 0) {
     const uint32_t run = 1u << a.xcd_run_log2;
     a.blocks_per_xcd = (a.blocks_per_xcd + run - 1) / run * run;
@@ -2775,9 +2775,10 @@ olbgfx_status launch_steps(olbgfx_lattice* L, uint32_t steps, hipStream_t stream
   }
   const dim3 grid(8 * a.blocks_per_xcd);
   const dim3 block(L->block_threads);
-  uint32_t lds = 0;
+  uint32_t waves = 0;
   int32_t order = -1;
-  default_launch(L, lds, order);
+  default_launch(L, waves, order);
+  const uint32_t lds = lds_for(L->block_threads, waves);
   int mode = L->uniform_id >= 0 ? L->table[L->uniform_id].kind : -1;
   if (L->boundary_kinds) {
     mode = kMaskedBoundary;
@@ -4128,8 +4129,22 @@ olbgfx_status olbgfx_set_launch(olbgfx_lattice* L, uint32_t block_threads, uint3
     return fail(OLBGFX_ERR_INVALID, "waves per SIMD must be in [0, 8]");
   }
   L->block_threads = block_threads;
-  L->lds_reserve = lds_for(block_threads, waves_per_simd);
+  L->waves = waves_per_simd;
   L->launch_given = true;
+  return OLBGFX_OK;
+}
+
+olbgfx_status olbgfx_get_launch(olbgfx_lattice* L, uint32_t* block_threads, uint32_t* waves_per_simd,
+                                int32_t* xcd_run_log2)
+{
+  if (check(L) != OLBGFX_OK || !block_threads || !waves_per_simd || !xcd_run_log2) {
+    return fail(OLBGFX_ERR_INVALID, "null argument");
+  }
+  if (prepare_boundary(L) != OLBGFX_OK) {
+    return OLBGFX_ERR_INVALID;
+  }
+  *block_threads = L->block_threads;
+  default_launch(L, *waves_per_simd, *xcd_run_log2);
   return OLBGFX_OK;
 }
 

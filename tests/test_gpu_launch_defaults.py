@@ -1,61 +1,28 @@
-"""What a lattice or an ensemble is launched with until a call sets it, against
-the settings the library offers: the default must not be the slower one.  Times
-are the least of alternating turns; the margins are half of the loss each rule
-was changed for."""
+"""What a lattice or an ensemble does until a call sets it: the launch of single
+steps on both sides of its rules, the runs that take two steps a pass, and that
+none of them is slower than what it replaces.  Times are compared on the same
+memory, in turns: two lattices of nearly the size of the Infinity Cache differ
+by up to a half with where their pages lie."""
 import time
 
 import numpy as np
 import pytest
 
-from openlb_amd import BGK, BOUNCE_BACK, FORCED_TRT, Dynamics, Ensemble, Lattice, cases
+from openlb_amd import (BGK, BOUNCE_BACK, FORCED_BGK, FORCED_TRT, SMAGORINSKY_BGK, TRT, Dynamics, Ensemble, Lattice,
+                        cases)
 
 pytestmark = pytest.mark.gpu
 
-
-def least(turns, repeats=6):
-    """the least time of each turn, the turns taken one after another"""
-    best = [np.inf] * len(turns)
-    for _ in range(repeats):
-        for k, turn in enumerate(turns):
-            t = time.perf_counter()
-            turn()
-            best[k] = min(best[k], time.perf_counter() - t)
-    return best
+BULK = {"bgk": Dynamics(BGK, omega=1 / 0.6), "trt": Dynamics(TRT, omega=1.3, magic=0.2),
+        "forced_bgk": Dynamics(FORCED_BGK, omega=1.3, force=(1e-5, 0.0, 0.0)),
+        "forced_trt": Dynamics(FORCED_TRT, omega=1.3, magic=0.2, force=(1e-5, 0.0, 0.0)),
+        "smagorinsky": Dynamics(SMAGORINSKY_BGK, omega=1 / 0.55, smagorinsky=0.12)}
 
 
-@pytest.mark.parametrize("res", [150, 170])
-def test_velocity_boundaries_take_no_occupancy_cap(res):
-    """a cap of 4 waves a SIMD costs 15 % at 150 and 10 % at 170"""
-    print(f"[launch defaults] LocalVelocity cavity {res}", flush=True)
-    case = cases.cavity3d_local_velocity(res, dtype=np.float32)
-    lats = []
-    for _ in range(2):
-        lat = Lattice(case.extent, case.padding, case.periodic, "f32")
-        case.apply(lat)
-        lats.append(lat)
-    lats[1].set_launch(256, 0)
-
-    def steps(lat):
-        for _ in range(20):
-            lat.collide_and_stream(1)
-        lat.synchronize()
-
-    for lat in lats:
-        steps(lat)
-    default, uncapped = least([lambda: steps(lats[0]), lambda: steps(lats[1])])
-    for lat in lats:
-        lat.close()
-    assert default <= (1.07 if res == 150 else 1.05) * uncapped
-
-
-BULK = {"bgk": Dynamics(BGK, omega=1 / 0.6), "forced_trt": Dynamics(FORCED_TRT, omega=1.3, magic=0.2,
-                                                                   force=(1e-5, 0.0, 0.0))}
-
-
-def _box(storage, kind, extent, padding):
-    """a uniform periodic box, one of BGK closed by bounce-back cells, or a
-    periodic one of ForcedTRT with oblique walls"""
-    lat = Lattice(extent, padding, (kind != "closed",) * 3, storage)
+def _box(storage, kind, extent, padding, periodic=True):
+    """a uniform box, one of BGK lined with bounce-back cells (closed unless
+    said otherwise), or one of ForcedTRT with oblique walls"""
+    lat = Lattice(extent, padding, (periodic and kind != "closed",) * 3, storage)
     mask = np.zeros(tuple(n + 2 * padding for n in extent), dtype=np.uint8)
     mask[tuple(slice(padding, -padding) for _ in range(3))] = 1
     lat.set_dynamics(1, BULK.get(kind, BULK["bgk"]))
@@ -72,66 +39,78 @@ def _box(storage, kind, extent, padding):
     return lat
 
 
-@pytest.mark.parametrize("storage,kind,extent", [("bf16", "bgk", (446, 87, 163)), ("f16", "bgk", (204, 125, 259)),
-                                                 ("f32", "porous", (116, 139, 227))])
-def test_single_steps_near_the_cache_size(storage, kind, extent):
-    """turns on short runs of blocks, which the cache does without (1.08 and
-    1.09), and a cap for masked cells of a periodic lattice (1.06)"""
-    print(f"[launch defaults] {storage} {kind} {extent} single steps", flush=True)
-    lats = [_box(storage, kind, extent, 1) for _ in range(2)]
-    lats[1].set_launch(256, 0)
-    lats[1].set_block_order(-1)
+@pytest.mark.parametrize("storage,kind,extent,periodic,waves,order", [
+    ("f32", "bgk", (140, 140, 140), True, 0, -1), ("f32", "bgk", (160, 160, 160), True, 4, -1),
+    ("f32", "trt", (160, 160, 160), False, 4, -1), ("f32", "smagorinsky", (160, 160, 160), True, 4, -1),
+    ("f32", "bgk", (256, 256, 256), True, 4, 4),
+    # the cap costs forced kinds up to 3 %, porous media 6 % (116x139x227)
+    ("f32", "forced_trt", (160, 160, 160), True, 0, -1), ("f32", "forced_bgk", (160, 160, 160), True, 0, -1),
+    ("f32", "porous", (116, 139, 227), True, 0, -1), ("f32", "closed", (160, 160, 160), True, 0, -1),
+    ("f32", "closed", (192, 192, 192), True, 4, -1), ("f32", "porous", (192, 192, 192), False, 4, -1),
+    # turns on short runs of blocks cost lattices in the cache 8 to 9 %
+    ("bf16", "bgk", (446, 87, 163), True, 0, -1), ("f16", "bgk", (204, 125, 259), True, 0, -1),
+    ("f16", "bgk", (220, 220, 220), True, 0, 3), ("f64", "bgk", (140, 140, 140), True, 0, -1)])
+def test_launch_of_single_steps(storage, kind, extent, periodic, waves, order):
+    print(f"[launch defaults] {storage} {kind} {extent}", flush=True)
+    lat = _box(storage, kind, extent, 1, periodic)
+    got = lat.get_launch()
+    lat.set_launch(128, 3)
+    lat.set_block_order(5)
+    given = lat.get_launch()
+    lat.close()
+    assert got == (256, waves, order)
+    assert given == (128, 3, 5)
 
-    def steps(lat):
-        for _ in range(40):
-            lat.collide_and_stream(1)
-        lat.synchronize()
 
-    for lat in lats:
-        steps(lat)
-    default, plain = least([lambda: steps(lats[0]), lambda: steps(lats[1])])
-    for lat in lats:
-        lat.close()
-    assert default <= 1.035 * plain
+@pytest.mark.parametrize("res", [150, 200])
+def test_velocity_boundaries_take_no_occupancy_cap(res):
+    """a cap of 4 waves a SIMD costs 15 % at 150 and 5 % at 200"""
+    print(f"[launch defaults] LocalVelocity cavity {res}", flush=True)
+    case = cases.cavity3d_local_velocity(res, dtype=np.float32)
+    lat = Lattice(case.extent, case.padding, case.periodic, "f32")
+    case.apply(lat)
+    got = lat.get_launch()
+    lat.close()
+    assert got == (256, 0, -1)
 
 
-# runs that took 1.08 to 1.2 of the single steps' time two steps a pass
+# runs that took 1.05 to 1.3 of the single steps' time two steps a pass
 LOSERS = [("f32", "bgk", (56, 56, 56), 1, 8), ("f32", "bgk", (145, 109, 171), 3, 20),
-          ("f32", "bgk", (206, 82, 165), 1, 5), ("f32", "bgk", (132, 155, 151), 3, 20), ("f64", "bgk", (123, 90, 129), 3, 8),
-          ("f64", "bgk", (547, 4, 547), 1, 5), ("f64", "closed", (5, 674, 674), 1, 20),
-          ("f16", "bgk", (1057, 1057, 8), 1, 20), ("f16", "bgk", (89, 522, 212), 1, 4), ("f16", "forced_trt", (1963, 1963, 4), 1, 8),
+          ("f32", "bgk", (206, 82, 165), 1, 5), ("f32", "bgk", (132, 155, 151), 3, 20),
+          ("f64", "bgk", (123, 90, 129), 3, 8), ("f64", "bgk", (547, 4, 547), 1, 5),
+          ("f64", "closed", (5, 674, 674), 1, 20), ("f16", "bgk", (1057, 1057, 8), 1, 20),
+          ("f16", "bgk", (89, 522, 212), 1, 4), ("f16", "forced_trt", (1963, 1963, 4), 1, 8),
           ("bf16", "forced_trt", (207, 227, 312), 1, 4), ("bf16", "forced_trt", (165, 245, 159), 3, 20)]
 
 
 @pytest.mark.parametrize("storage,kind,extent,padding,steps", LOSERS)
 def test_runs_are_not_slower_than_single_steps(storage, kind, extent, padding, steps):
     print(f"[launch defaults] {storage} {kind} {extent} runs of {steps}", flush=True)
-    lats = [_box(storage, kind, extent, padding) for _ in range(2)]
-    lats[1].set_two_step(0)
-    cells = int(np.prod(extent))
-    calls = max(2, int(2e8 / (cells * steps)))
-
-    def run(lat):
+    lat = _box(storage, kind, extent, padding)
+    calls = max(2, int(2e8 / (int(np.prod(extent)) * steps)))
+    best = [np.inf, np.inf]
+    for turn in range(8):
+        single = turn % 2
+        lat.set_two_step(0 if single else None)
+        lat.collide_and_stream(steps)
+        lat.synchronize()
+        t = time.perf_counter()
         for _ in range(calls):
             lat.collide_and_stream(steps)
         lat.synchronize()
-
-    for lat in lats:
-        run(lat)
-    default, single = least([lambda: run(lats[0]), lambda: run(lats[1])])
-    for lat in lats:
-        lat.close()
-    assert default <= 1.045 * single
+        best[single] = min(best[single], time.perf_counter() - t)
+    lat.close()
+    assert best[0] <= 1.045 * best[1]
 
 
 @pytest.mark.parametrize("storage,kind,extent,padding,steps,pairs", [
     ("f32", "bgk", (44, 44, 44), 1, 4, 4), ("f32", "bgk", (64, 64, 64), 3, 7, 4), ("f32", "bgk", (101, 101, 101), 1, 8, 8),
     ("f32", "bgk", (160, 160, 160), 3, 5, 4), ("f32", "closed", (160, 160, 160), 1, 4, 4),
-    ("f64", "bgk", (72, 72, 72), 1, 4, 4), ("f64", "bgk", (94, 94, 94), 1, 13, 12), ("f64", "bgk", (140, 140, 140), 1, 4, 4),
-    ("f16", "bgk", (220, 220, 220), 1, 9, 8), ("f16", "forced_trt", (193, 193, 193), 1, 4, 4),
-    ("bf16", "bgk", (193, 193, 193), 1, 4, 4), ("bf16", "forced_trt", (344, 250, 86), 1, 12, 12),
-    ("f64", "bgk", (94, 94, 94), 1, 11, 0), ("f16", "bgk", (220, 220, 220), 1, 7, 0),
-    ("bf16", "forced_trt", (344, 250, 86), 1, 11, 0)])
+    ("f64", "bgk", (72, 72, 72), 1, 4, 4), ("f64", "bgk", (97, 97, 97), 1, 13, 12), ("f64", "bgk", (140, 140, 140), 1, 4, 4),
+    ("f64", "bgk", (97, 97, 97), 1, 11, 0),
+    ("f16", "bgk", (220, 220, 220), 1, 9, 8), ("f16", "bgk", (220, 220, 220), 1, 7, 0),
+    ("f16", "forced_trt", (193, 193, 193), 1, 4, 4), ("bf16", "bgk", (193, 193, 193), 1, 4, 4),
+    ("bf16", "forced_trt", (344, 250, 86), 1, 12, 12), ("bf16", "forced_trt", (344, 250, 86), 1, 11, 0)])
 def test_steps_taken_two_a_pass(storage, kind, extent, padding, steps, pairs):
     """both sides of the rules"""
     print(f"[launch defaults] {storage} {kind} {extent} {steps} steps", flush=True)
@@ -148,29 +127,24 @@ def test_small_ensembles_take_no_occupancy_cap(storage):
     """single steps of 4 cavities 64^3, which the cache holds: the cap for
     ensembles that it does not hold costs 7 %"""
     print(f"[launch defaults] ensemble {storage}", flush=True)
-    enss, lats = [], []
-    for _ in range(2):
-        group = []
-        for _ in range(4):
-            case = cases.box_cavity(64, dtype=np.float32)
-            lat = Lattice(case.extent, case.padding, case.periodic, storage)
-            case.apply(lat)
-            group.append(lat)
-        enss.append(Ensemble(group))
-        lats.append(group)
-    enss[1].set_launch(256, 0, 1)
-
-    def steps(k):
+    lats = []
+    for _ in range(4):
+        case = cases.box_cavity(64, dtype=np.float32)
+        lat = Lattice(case.extent, case.padding, case.periodic, storage)
+        case.apply(lat)
+        lats.append(lat)
+    both = [Ensemble(lats), Ensemble(lats)]  # of the same lattices
+    both[1].set_launch(256, 0, 1)
+    best = [np.inf, np.inf]
+    for turn in range(16):
+        ens = both[turn % 2]
+        ens.step(1)
+        lats[0].synchronize()
+        t = time.perf_counter()
         for _ in range(50):
-            enss[k].step(1)
-        lats[k][0].synchronize()
-
-    for k in (0, 1):
-        steps(k)
-    default, uncapped = least([lambda: steps(0), lambda: steps(1)], 8)
-    for ens in enss:
-        ens.close()
-    for group in lats:
-        for lat in group:
-            lat.close()
-    assert default <= 1.035 * uncapped
+            ens.step(1)
+        lats[0].synchronize()
+        best[turn % 2] = min(best[turn % 2], time.perf_counter() - t)
+    for x in (*both, *lats):
+        x.close()
+    assert best[0] <= 1.035 * best[1]
