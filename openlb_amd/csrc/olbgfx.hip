@@ -2417,7 +2417,8 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
 // in the cache: FP32 64^3 8.5 / 7.2, 101^3 27.5 / 16.6; FP64 64^3 14.3 / 11.9,
 // 100^3 43.5 / 41.  Between the two the second set drives the first out: FP32
 // boxes of 2.4 to 3.0 M cells take 0.86 to 1.24 of the single step's time, FP64
-// boxes of 180 to 255 MiB 0.9 to 1.17.  Masked cells and Smagorinsky BGK in
+// boxes with 176 MiB of core populations and more, up to 260 in all, 0.77 to
+// 1.17.  Masked cells and Smagorinsky BGK in
 // 2-byte storage are bound by instruction issue: the former lose (porous
 // channel FP16 124 / 133), the latter gain 7 % in long runs and lose 8 % in runs
 // of 8 steps, whose first and last pass convert the layout.
@@ -2431,7 +2432,7 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
   const bool masked = mode < 0 || mode >= kWithWalls;
   const olbgfx_lattice_desc& D = L->desc;
   const uint64_t cells = (uint64_t)D.nx * D.ny * D.nz;
-  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
+  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20, core = (Q * cells * L->elem) >> 20;
   const bool bgk = mode == OLBGFX_BGK;
   if (L->elem == 2) {
     // BF16 ForcedTRT still gains from the cache at 257 MiB (165x245x159 1.18)
@@ -2442,7 +2443,7 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
     return cells >= (64u << 20) || (bgk && L->desc.storage == OLBGFX_STORE_BF16) ? 512 : 1024;
   }
   if (L->elem == 8) {
-    return mib >= 260 || (bgk && mib >= 48 && mib < 176) ? 512 : 0;
+    return mib >= 260 || (bgk && mib >= 48 && core < 176) ? 512 : 0;
   }
   if (bgk && cells < 1500000) {
     return cells >= 60000 ? 512 : 0;
@@ -2463,9 +2464,11 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
 //   7.2 / 8.1, but 44^3 6.0 / 5.1 and 52^3 6.8 / 6.4, whose tiles sweep a single
 //   plane with one workgroup a CU, or with enough cells for two.  Up to 400000
 //   cells in tiles of three planes and more, runs of 5 steps up to 1.04.
-// - FP64 from 128 to 176 MiB runs of 5 steps 1.04, of 9 1.03, of 12 and more 0.73
-//   to 0.98; up to 340 MiB other kinds than BGK 1.05 in runs of 5 steps, BGK on
-//   lattices thin along x or y 1.16.
+// - FP64 BGK with 126 to 150 MiB of core populations, runs of 5 steps 1.04, of 9
+//   1.03, of 12 and more 0.73 to 0.98; with 150 to 176 MiB of 5 1.08, of 15 1.03,
+//   of 20 and more 0.84 to 1.00; above that up to 1.09.  Up to 340 MiB other
+//   kinds than BGK 1.05 in runs of 5 steps, BGK on lattices thin along x or y
+//   1.16.
 // - FP64 ForcedTRT above 3.0 turns 1.02 to 1.11, general masks above 2.8 turns
 //   1.02 to 1.13.
 // - Closed lattices thin along x or y, whose padding planes are updated too:
@@ -2479,7 +2482,7 @@ bool pair_pays(const olbgfx_lattice* L, int mode, const PairPlan& plan, uint32_t
 {
   const olbgfx_lattice_desc& D = L->desc;
   const uint64_t cells = (uint64_t)D.nx * D.ny * D.nz;
-  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
+  const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20, core = (Q * cells * L->elem) >> 20;
   const bool bgk = mode == OLBGFX_BGK, forced = mode == OLBGFX_FORCED_TRT;
   const bool thin = D.nx < 16 || D.ny < 16;
   if (!plan.worth || (thin && !D.periodic[0])) {
@@ -2496,7 +2499,7 @@ bool pair_pays(const olbgfx_lattice* L, int mode, const PairPlan& plan, uint32_t
   }
   if (L->elem == 8) {
     if (mib < 260) {
-      return mib < 128 || steps >= 12;
+      return steps >= (core < 126 ? 4u : core < 150 ? 12u : 20u);
     }
     return (mib >= 340 || (!thin && (bgk || steps >= 12))) && plan.turns <= (mode < 0 ? 2.8 : forced ? 3.0 : 1e9);
   }

@@ -107,7 +107,8 @@ def test_runs_are_not_slower_than_single_steps(storage, kind, extent, padding, s
     ("f32", "bgk", (44, 44, 44), 1, 4, 4), ("f32", "bgk", (64, 64, 64), 3, 7, 4), ("f32", "bgk", (101, 101, 101), 1, 8, 8),
     ("f32", "bgk", (160, 160, 160), 3, 5, 4), ("f32", "closed", (160, 160, 160), 1, 4, 4),
     ("f64", "bgk", (72, 72, 72), 1, 4, 4), ("f64", "bgk", (97, 97, 97), 1, 13, 12), ("f64", "bgk", (140, 140, 140), 1, 4, 4),
-    ("f64", "bgk", (97, 97, 97), 1, 11, 0),
+    ("f64", "bgk", (97, 97, 97), 1, 11, 0), ("f64", "bgk", (92, 108, 115), 3, 20, 20),
+    ("f64", "bgk", (92, 108, 115), 3, 19, 0),
     ("f16", "bgk", (220, 220, 220), 1, 9, 8), ("f16", "bgk", (220, 220, 220), 1, 7, 0),
     ("f16", "forced_trt", (193, 193, 193), 1, 4, 4), ("bf16", "bgk", (193, 193, 193), 1, 4, 4),
     ("bf16", "forced_trt", (344, 250, 86), 1, 12, 12), ("bf16", "forced_trt", (344, 250, 86), 1, 11, 0)])
