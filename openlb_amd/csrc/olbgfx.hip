@@ -2416,7 +2416,7 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
 // they win only for uniform BGK, and there while both sets of populations lie
 // in the cache: FP32 64^3 8.5 / 7.2, 101^3 27.5 / 16.6; FP64 64^3 14.3 / 11.9,
 // 100^3 43.5 / 41.  Between the two the second set drives the first out: FP32
-// boxes of 2.4 to 3.0 M cells take 0.86 to 1.24 of the single step's time, FP64
+// boxes of 2.4 to 3.3 M cells take 0.86 to 1.24 of the single step's time, FP64
 // boxes with 176 MiB of core populations and more, up to 260 in all, 0.77 to
 // 1.17.  Masked cells and Smagorinsky BGK in
 // 2-byte storage are bound by instruction issue: the former lose (porous
@@ -2448,7 +2448,7 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
   if (bgk && cells < 1500000) {
     return cells >= 60000 ? 512 : 0;
   }
-  return mib >= 256 ? 1024 : 0;
+  return mib >= 256 || (bgk && cells >= 2400000) ? 1024 : 0;
 }
 
 // Do runs that take `steps` steps (a multiple of four) in pairs win with these
@@ -2464,6 +2464,9 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
 //   7.2 / 8.1, but 44^3 6.0 / 5.1 and 52^3 6.8 / 6.4, whose tiles sweep a single
 //   plane with one workgroup a CU, or with enough cells for two.  Up to 400000
 //   cells in tiles of three planes and more, runs of 5 steps up to 1.04.
+// - FP32 BGK from 2.4 M cells to 256 MiB: where one workgroup a CU takes tiles as
+//   wide as the rows, runs of 20 steps 0.87 to 0.98, of 15 up to 1.00, of 5 up to
+//   1.10 (26 boxes); with more tiles a row 0.91 to 1.17 in runs of any length.
 // - FP64 BGK with 126 to 150 MiB of core populations, runs of 5 steps 1.04, of 9
 //   1.03, of 12 and more 0.73 to 0.98; with 150 to 176 MiB of 5 1.08, of 15 1.03,
 //   of 20 and more 0.84 to 1.00; above that up to 1.09.  Up to 340 MiB other
@@ -2506,6 +2509,9 @@ bool pair_pays(const olbgfx_lattice* L, int mode, const PairPlan& plan, uint32_t
   if (plan.threads == 512) {
     return cells >= 220000 ? cells >= 400000 || plan.xlen < 3 || steps >= 8
                            : plan.xlen == 1 && (plan.nwork <= 256 || cells >= 135000);
+  }
+  if (mib < 256) {
+    return steps >= 12 && plan.ntz == 1 && plan.nwork <= 256;
   }
   return plan.turns <= 3.0;
 }

@@ -105,7 +105,8 @@ def test_runs_are_not_slower_than_single_steps(storage, kind, extent, padding, s
 
 @pytest.mark.parametrize("storage,kind,extent,padding,steps,pairs", [
     ("f32", "bgk", (44, 44, 44), 1, 4, 4), ("f32", "bgk", (64, 64, 64), 3, 7, 4), ("f32", "bgk", (101, 101, 101), 1, 8, 8),
-    ("f32", "bgk", (160, 160, 160), 3, 5, 4), ("f32", "closed", (160, 160, 160), 1, 4, 4),
+    ("f32", "bgk", (140, 140, 140), 1, 14, 12), ("f32", "bgk", (140, 140, 140), 1, 11, 0),
+    ("f32", "bgk", (153, 113, 171), 3, 40, 0), ("f32", "bgk", (160, 160, 160), 3, 5, 4), ("f32", "closed", (160, 160, 160), 1, 4, 4),
     ("f64", "bgk", (72, 72, 72), 1, 4, 4), ("f64", "bgk", (97, 97, 97), 1, 13, 12), ("f64", "bgk", (140, 140, 140), 1, 4, 4),
     ("f64", "bgk", (97, 97, 97), 1, 11, 0), ("f64", "bgk", (92, 108, 115), 3, 20, 20),
     ("f64", "bgk", (92, 108, 115), 3, 19, 0),
