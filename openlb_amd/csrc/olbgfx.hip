@@ -2140,8 +2140,9 @@ uint32_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
 // 538 / 497, FP16 279 / 263; 256^3 FP32 550 / 509, cavity 552 / 509, FP64 1051
 // / 1018.  Between 256 MiB and 1 GiB contiguous parts stay better in 4-byte
 // storage (40x300x400 capped: 138 against 144, 150 without the cap), and below
-// 256 MiB the cache serves them best (160^3 FP16 47 against 49, 446x87x163 BF16
-// of 238 MiB 65 against 70, cavity 33^3 FP32 4.8 against 5.3).
+// that, in 2-byte storage below 250 MiB, the cache serves them best (160^3 FP16
+// 47 against 49, 446x87x163 BF16 of 238 MiB 65 against 70, but 88x149x468 FP16 of
+// 250 MiB 85 against 80; cavity 33^3 FP32 4.8 against 5.3).
 // The cap is for kernels with registers for more than 4 waves that wait for
 // memory alone: BGK, TRT and Smagorinsky on 60 random boxes of 256 to 480 MiB
 // 0.89 to 0.99 of the time without, but forced kinds 0.98 to 1.03, masked cells
@@ -2160,7 +2161,7 @@ void default_launch(const olbgfx_lattice* L, uint32_t& waves, int32_t& order)
   if (L->order_given) {
     order = L->xcd_run_log2;
   } else if (L->elem == 2) {
-    order = mib >= 256 ? 3 : -1;
+    order = mib >= 250 ? 3 : -1;
   } else {
     order = mib >= 1024 ? 4 : -1;
   }
