@@ -2147,8 +2147,9 @@ uint32_t lds_for(uint32_t block_threads, uint32_t waves_per_simd)
 // memory alone: BGK, TRT and Smagorinsky on 60 random boxes of 256 to 480 MiB
 // 0.89 to 0.99 of the time without, but forced kinds 0.98 to 1.03, masked cells
 // on periodic lattices up to 1.06 (others 0.95 to 1.05, from 512 MiB 0.95 to
-// 1.00), and velocity and pressure boundaries, which hide their chains of loads behind other waves,
-// more (LocalVelocity cavity, 150^3 162 against 141 us, 200^3 331 / 314).
+// 1.00), and velocity and pressure boundaries, which hide their chains of loads
+// behind other waves, more (LocalVelocity cavity, 150^3 162 against 141 us,
+// 200^3 331 / 314).
 void default_launch(const olbgfx_lattice* L, uint32_t& waves, int32_t& order)
 {
   const uint64_t mib = ((uint64_t)Q * L->stride * L->elem) >> 20;
@@ -2418,7 +2419,7 @@ olbgfx_status prepare_split(olbgfx_lattice* L)
 // in the cache: FP32 64^3 8.5 / 7.2, 101^3 27.5 / 16.6; FP64 64^3 14.3 / 11.9,
 // 100^3 43.5 / 41.  Between the two the second set drives the first out: FP32
 // boxes of 2.4 to 3.3 M cells take 0.86 to 1.24 of the single step's time, FP64
-// boxes with 176 MiB of core populations and more, up to 260 in all, 0.77 to
+// boxes with 170 MiB of core populations and more, up to 260 in all, 0.77 to
 // 1.17.  Masked cells and Smagorinsky BGK in
 // 2-byte storage are bound by instruction issue: the former lose (porous
 // channel FP16 124 / 133), the latter gain 7 % in long runs and lose 8 % in runs
@@ -2444,7 +2445,7 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
     return cells >= (64u << 20) || (bgk && L->desc.storage == OLBGFX_STORE_BF16) ? 512 : 1024;
   }
   if (L->elem == 8) {
-    return mib >= 260 || (bgk && mib >= 48 && core < 176) ? 512 : 0;
+    return mib >= 260 || (bgk && mib >= 48 && core < 170) ? 512 : 0;
   }
   if (bgk && cells < 1500000) {
     return cells >= 60000 ? 512 : 0;
@@ -2469,10 +2470,10 @@ uint32_t pair_threads(const olbgfx_lattice* L, int mode)
 //   wide as the rows, runs of 20 steps 0.87 to 0.98, of 15 up to 1.00, of 5 up to
 //   1.10 (26 boxes); with more tiles a row 0.91 to 1.17 in runs of any length.
 // - FP64 BGK with 126 to 150 MiB of core populations, runs of 5 steps 1.04, of 9
-//   1.03, of 12 and more 0.73 to 0.98; with 150 to 176 MiB of 5 1.08, of 15 1.03,
+//   1.03, of 12 and more 0.73 to 0.98; with 150 to 170 MiB of 5 1.08, of 15 1.03,
 //   of 20 and more 0.84 to 1.00; above that up to 1.09.  Up to 340 MiB other
-//   kinds than BGK 1.05 in runs of 5 steps, BGK on lattices thin along x or y
-//   1.16.
+//   kinds than BGK 1.05 in runs of 5 steps, general masks below 300 MiB 1.06 in
+//   runs of any length, BGK on lattices thin along x or y 1.16.
 // - FP64 ForcedTRT above 3.0 turns 1.02 to 1.11, general masks above 2.8 turns
 //   1.02 to 1.13.
 // - Closed lattices thin along x or y, whose padding planes are updated too:
@@ -2505,7 +2506,8 @@ bool pair_pays(const olbgfx_lattice* L, int mode, const PairPlan& plan, uint32_t
     if (mib < 260) {
       return steps >= (core < 126 ? 4u : core < 150 ? 12u : 20u);
     }
-    return (mib >= 340 || (!thin && (bgk || steps >= 12))) && plan.turns <= (mode < 0 ? 2.8 : forced ? 3.0 : 1e9);
+    const bool large = mib >= 340 || (!thin && (bgk || (steps >= 12 && (mode >= 0 || mib >= 300))));
+    return large && plan.turns <= (mode < 0 ? 2.8 : forced ? 3.0 : 1e9);
   }
   if (plan.threads == 512) {
     return cells >= 220000 ? cells >= 400000 || plan.xlen < 3 || steps >= 8
